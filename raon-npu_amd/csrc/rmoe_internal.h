@@ -417,6 +417,11 @@ hipError_t launch_synth_quantize(uint64_t seed, float std, int M, int K, int k_v
 hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y, RmoeScratch& s,
                          hipStream_t st);
 
+// Both formats on MFMA (linear_mfma.hip), for the operands linear_mfma_ok() accepts.
+bool linear_mfma_ok(int M, int K, const uint16_t* x, int T, const uint16_t* y);
+hipError_t launch_linear_mfma(const uint8_t* tiles, int fmt, int M, int K, const uint16_t* x, int T, uint16_t* y,
+                              hipStream_t st);
+
 // bfp16ebs8 (bfp16_gemv.hip).  The GEMV splits K over bfp16_ksplit(M, K) workgroups
 // (at most (K/128 + 3)/4, so the q4nx scratch sizing covers it).
 hipError_t launch_b16_relayout_in(const uint8_t* packed, uint8_t* tiles, int M, int K, hipStream_t st);

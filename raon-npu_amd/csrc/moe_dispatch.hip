@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __
                                                                int32_t* __restrict__ offsets,
                                                                int32_t* __restrict__ order, int32_t* __restrict__ inv,
                                                                uint32_t* __restrict__ tiles, int* __restrict__ ntiles,
-                                                               int cap, int shared_rows) {
+                                                               int cap, int shared_rows, int bm) {
   __shared__ int slot[4][256];  // per wave: counts, then next output slot per expert
   __shared__ int wsum[4];
   const int c = blockIdx.x, tid = threadIdx.x, wave = wave_id(), lane = tid & 63;
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __
     __shared__ int tsum[kTileClasses][4];
     const int ng = E + (shared_rows > 0 ? 1 : 0);
     const int gb = tid < E ? offset : n;
-    tile_table_block<4>(tid, ng, gb, gb + (tid < E ? total : shared_rows), tiles, ntiles, cap, tsum);
+    tile_table_block<4>(tid, ng, gb, gb + (tid < E ? total : shared_rows), tiles, ntiles, cap, bm, tsum);
   }
 }
 
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __
 
 hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int32_t* order, int32_t* inv,
                            int32_t* offsets, RmoeScratch& s, hipStream_t st, uint32_t* tiles, int* ntiles, int cap,
-                           int shared_rows, bool counted) {
+                           int shared_rows, bool counted, int bm) {
   const int n = T * k;
   const int nchunks = (n + kChunk - 1) / kChunk;
   if (n_experts < 1 || n_experts > 256) return hipErrorInvalidValue;
@@ -157,7 +157,7 @@ hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int3
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(dispatch_scatter_kernel, dim3(nchunks), dim3(256), 0, st, ids, n, n_experts, s.chunk_counts,
-                     nchunks, offsets, order, inv, tiles, ntiles, cap, shared_rows);
+                     nchunks, offsets, order, inv, tiles, ntiles, cap, shared_rows, bm);
   return hipGetLastError();
 }
 

@@ -16,8 +16,11 @@
 // exponents are undone exactly in fp32.  The correction (second sum) is a small GEMM over
 // the groups on bf16 MFMA: min and 8*scale are exact bf16 values and S is split exactly
 // into three bf16 parts, so its six products are the whole correction.
+#include <algorithm>
+
 #include "../../include/raon_moe.h"
 #include "rmoe_internal.h"
+#include "wave_gemm.h"
 
 namespace rmoe {
 namespace {
@@ -439,7 +442,7 @@ __global__ __launch_bounds__(256) void router_prep_kernel(const uint16_t* __rest
 // cases and the table for a second GEMM with other shared rows.)
 __global__ __launch_bounds__(512) void tile_table_kernel(const int32_t* __restrict__ offsets, int n_routed,
                                                          int shared_base, int shared_rows, uint32_t* __restrict__ tiles,
-                                                         int* __restrict__ ntiles, int cap) {
+                                                         int* __restrict__ ntiles, int cap, int bm) {
   __shared__ int wsum[kTileClasses][8];
   const int e = threadIdx.x;
   const int ng = n_routed + (shared_rows > 0 ? 1 : 0);
@@ -448,7 +451,7 @@ __global__ __launch_bounds__(512) void tile_table_kernel(const int32_t* __restri
     b = e < n_routed ? offsets[e] : shared_base;
     end = e < n_routed ? offsets[e + 1] : shared_base + shared_rows;
   }
-  tile_table_block<8>(e, ng, b, end, tiles, ntiles, cap, wsum);
+  tile_table_block<8>(e, ng, b, end, tiles, ntiles, cap, bm, wsum);
 }
 
 // ------------------------------------------------------------- grouped GEMM --
@@ -483,6 +486,8 @@ struct GemmArgs {
   // bfp16 weights (down of a weights-d layer): per expert and weight row the largest
   // max(e, 7) of the row's blocks ([experts][N_total]).
   const uint8_t* rowexp;
+  // mode 1, few rows: exponents of the src rows per 128-column chunk [rows][exp_stride(K)].
+  const int8_t* hexp;
   // mode 1: D rows are stored with the non-temporal hint (a large D, read once by the
   // combine, then stays out of the caches the GEMM reuses weights and rows from).
   int out_nt;
@@ -490,6 +495,11 @@ struct GemmArgs {
 
 __device__ __forceinline__ int group_end(const GemmArgs& a, int e) {
   return e < a.n_routed ? a.offsets[e + 1] : a.shared_base + a.shared_rows;
+}
+
+// A shared tile in a GEMM without shared rows (gate/up with the shared gate/up given).
+__device__ __forceinline__ bool skip_tile(const GemmArgs& a, uint32_t te) {
+  return a.shared_rows == 0 && (int)(te & 511u) == a.n_routed;
 }
 
 // LDS ring of the grouped GEMM: per K step (128 columns) the workgroup's 128 activation
@@ -1294,6 +1304,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (lid >= n) return;
   const int mt = lid / a.n_tiles, nt = lid % a.n_tiles;
   const uint32_t* tl = a.tiles + (size_t)c * cap;
+  if (skip_tile(a, tl[mt])) return;
   if constexpr (kB16) {
     if (c == 2) gemm_tile_b16<class_fragments(2)>(a, tl, mt, nt, lds, rowidx, row_e);
     else if (c == 1) gemm_tile_b16<class_fragments(1)>(a, tl, mt, nt, lds, rowidx, row_e);
@@ -1310,6 +1321,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 }
+
+#include "few_rows_gemm.h"
 
 // ---------------------------------------------------------------- combine --
 // out[t] = RTNE(RTNE(sum_{routes by ascending expert} f32(D[inv[t,r]]) * w[t,r]) + D_shared[t])
@@ -1539,21 +1552,46 @@ hipError_t launch_topk(const float* logits, int T, int E, int k, int score, cons
 // for the worst case (a class-0/1 tile is a group's last, so at most one per group),
 // 8 x ceil(tiles / 8) workgroups per class (the XCD mapping deals each class in eighths).
 static hipError_t launch_grouped(GemmArgs a, uint32_t* tiles, int* ntiles, int cap, int n_routed, hipStream_t st,
-                                 bool b16 = false) {
+                                 bool b16, bool few) {
   a.tiles = tiles;
   a.ntiles = ntiles;
   const int small = min(cap, n_routed + 1);
-  const int blocks = 8 * ((a.n_tiles * cap + 7) / 8 + 2 * ((a.n_tiles * small + 7) / 8));
-  if (b16)
-    hipLaunchKernelGGL((grouped_gemm_kernel<7, true>), dim3(blocks), dim3(512), 0, st, a, cap);
-  else
-    hipLaunchKernelGGL((grouped_gemm_kernel<7, false>), dim3(blocks), dim3(512), 0, st, a, cap);
+  const int per2 = 8 * ((a.n_tiles * cap + 7) / 8), per01 = 8 * ((a.n_tiles * small + 7) / 8);
+  if (few) {
+    const dim3 grid(per2 + 2 * per01), block(256);
+    if (a.mode == 0)
+      hipLaunchKernelGGL((few_rows_gemm_kernel<false, false>), grid, block, 0, st, a, cap);
+    else if (b16)
+      hipLaunchKernelGGL((few_rows_gemm_kernel<true, true>), grid, block, 0, st, a, cap);
+    else
+      hipLaunchKernelGGL((few_rows_gemm_kernel<true, false>), grid, block, 0, st, a, cap);
+  } else if (b16) {
+    hipLaunchKernelGGL((grouped_gemm_kernel<7, true>), dim3(per2 + 2 * per01), dim3(512), 0, st, a, cap);
+  } else {
+    hipLaunchKernelGGL((grouped_gemm_kernel<7, false>), dim3(per2 + 2 * per01), dim3(512), 0, st, a, cap);
+  }
   return hipGetLastError();
+}
+
+// Whether the batch's groups are short enough for few_rows_gemm_kernel: on average at most
+// kFewRows assignments per routed expert.  The line lies where the groups start to need a
+// second 48-row tile.  Whole layer, few-rows against grouped_gemm_kernel: H=2048, I=768, 8
+// of 128 experts: 8 tokens 71 / 88 us, 445 148 / 163, 640 (40 rows) 161 / 192, 800 (50) 206 /
+// 200, 1,024 248 / 236; H=2560, I=1088, 6 of 128: 300 tokens 214 / 259, 1,000 (47 rows) 346 /
+// 358, 2,000 576 / 560.
+constexpr int kFewRows = 46;
+static bool few_rows(size_t assignments, int n_routed) { return assignments <= (size_t)kFewRows * n_routed; }
+// Tiles of a class at most: the full ones and one remainder per group.
+static size_t tile_capacity(const RmoeLayer& L, int T) {
+  const size_t A = (size_t)T * L.top_k;
+  const int bm = few_rows(A, L.n_routed) ? kBMFew : kBM;
+  return A / bm + L.n_routed + T / bm + 4;
 }
 
 size_t prefill_scratch_bytes(const RmoeLayer& L, int T) {
   const size_t A = (size_t)T * L.top_k, R = A + T;
-  const size_t tiles = A / kBM + L.n_routed + T / kBM + 4;
+  const size_t tiles = std::max(A / kBM + T / kBM, std::min<size_t>(A, (size_t)kFewRows * L.n_routed) / kBMFew + T / kBMFew) +
+                       L.n_routed + 4;
   return R * L.Ipad * 2                                  // h (fp16 operand)
          + R * 3 * sum_planes_gp(L.Ipad / 32) * 2        // h group sums
          + R * exp_stride(L.Ipad) + R                    // h exponents (per chunk, per row)
@@ -1593,7 +1631,8 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   int8_t* xexp = (int8_t*)carve((size_t)T);
   uint16_t* xsum = (uint16_t*)carve((size_t)T * 3 * Gpx * 2);
   float* logits = (float*)carve((size_t)T * E * 16);
-  const int tile_cap = (int)(A / kBM + E + T / kBM + 4);
+  const bool few = few_rows(A, E);
+  const int bm = few ? kBMFew : kBM, tile_cap = (int)tile_capacity(L, T);
   uint32_t* tiles = (uint32_t*)carve((size_t)kTileClasses * tile_cap * 4);
   int* ntiles = (int*)carve(256);
   hipError_t err;
@@ -1617,11 +1656,11 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
     hipLaunchKernelGGL(prep_x_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, x, T, L.H, xh, xexp, xsum);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
-  // The gate/up GEMM's groups: routed, and the shared expert unless its gate/up is given.
-  const int gu_shared_rows = shared_gu ? 0 : T;
-  const bool fused_table = E + (gu_shared_rows > 0 ? 1 : 0) <= 256;
-  err = fused_table ? launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, tiles, ntiles, tile_cap,
-                                      gu_shared_rows, counted)
+  // One tile table for both GEMMs: the routed groups and the shared one, whose tiles the
+  // gate/up GEMM skips when its gate/up is given.
+  const bool fused_table = E + 1 <= 256;
+  err = fused_table ? launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, tiles, ntiles, tile_cap, T,
+                                      counted, bm)
                     : launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, nullptr, nullptr, 0, 0, counted);
   if (err != hipSuccess) return err;
   if (L.Ipad > L.I) {
@@ -1650,7 +1689,7 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   g.tiles = tiles;
   g.ntiles = ntiles;
   g.offsets = s.offsets;
-  g.shared_rows = gu_shared_rows;
+  g.shared_rows = shared_gu ? 0 : T;
   g.out = h;
   g.out_ld = L.Ipad;
   g.out_ssum = hsum;
@@ -1659,8 +1698,8 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   g.gb = gb;
   g.vb = vb;
   if (!fused_table) {
-    hipLaunchKernelGGL(tile_table_kernel, dim3(1), dim3(512), 0, st, s.offsets, E, (int)A, g.shared_rows, tiles,
-                       ntiles, tile_cap);
+    hipLaunchKernelGGL(tile_table_kernel, dim3(1), dim3(512), 0, st, s.offsets, E, (int)A, T, tiles, ntiles,
+                       tile_cap, bm);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   if (shared_gu) {
@@ -1669,16 +1708,13 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
                        L.Ipad, act, gb, vb, h + A * L.Ipad, hsum + A * 3 * Gph, hexp + A * exp_stride(L.Ipad));
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
-  if ((err = launch_grouped(g, tiles, ntiles, tile_cap, E, st)) != hipSuccess) return err;
-  hipLaunchKernelGGL(h_unify_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, h, hexp, (int)R, L.Ipad,
-                     hrow);
-  if ((err = hipGetLastError()) != hipSuccess) return err;
-  // Down: every sorted row (routed + shared), rows of h contiguous.
-  if (shared_gu) {
-    hipLaunchKernelGGL(tile_table_kernel, dim3(1), dim3(512), 0, st, s.offsets, E, (int)A, T, tiles, ntiles,
-                       tile_cap);
+  if ((err = launch_grouped(g, tiles, ntiles, tile_cap, E, st, false, few)) != hipSuccess) return err;
+  if (!few) {  // few_rows_tile takes the chunks' exponents itself
+    hipLaunchKernelGGL(h_unify_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, h, hexp, (int)R, L.Ipad,
+                       hrow);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
+  // Down: every sorted row (routed + shared), rows of h contiguous.
   GemmArgs d = g;
   d.wbase = L.dn;
   d.wstride = L.dn_bytes;
@@ -1688,6 +1724,7 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   d.n_tiles = L.H / 256;
   d.src = h;
   d.aexp = hrow;
+  d.hexp = hexp;
   d.ssum = hsum;
   d.shared_rows = T;
   d.out = D;
@@ -1699,7 +1736,7 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   // (247 MB of D), but 0.170 -> 0.171 ms at 445 tokens (16 MB), where the combine finds
   // more of D in the caches.
   d.out_nt = R * (size_t)L.H * 2 > ((size_t)64 << 20) ? 1 : 0;
-  if ((err = launch_grouped(d, tiles, ntiles, tile_cap, E, st, L.dn_fmt == RMOE_FMT_BFP16)) != hipSuccess) return err;
+  if ((err = launch_grouped(d, tiles, ntiles, tile_cap, E, st, L.dn_fmt == RMOE_FMT_BFP16, few)) != hipSuccess) return err;
   hipLaunchKernelGGL(combine_kernel, dim3(T), dim3(256), 0, st, D, L.H, ids, wts, s.inv, k, E, (int)A,
                      residual ? x : nullptr, out, routed, shared_down, 1);
   return hipGetLastError();

@@ -251,15 +251,22 @@ __device__ __forceinline__ bool arrive_last(unsigned* counter, unsigned n, unsig
 }
 
 // ---- grouped GEMM tile table ----
-// The m-tiles of every group of expert-sorted rows, 128 rows each; a tile is
+// The m-tiles of every group of expert-sorted rows, bm rows each; a tile is
 // group | (row_start << 9).  Tiles are listed by class, the number of 16-row fragments
-// that hold rows: class 0 (up to 32 rows: 2 fragments), 1 (up to 64: 4), 2 (8); the
-// grouped GEMM runs each class with that many fragments, so a group's short last tile
-// does no MFMA work on absent rows.  Class c's tiles sit at tiles[c * cap ...] in group
-// order, their count in ntiles[c].
+// that hold rows, so that a group's short last tile does no MFMA work on absent rows.
+//   bm = kBM (128): class 0 (up to 32 rows: 2 fragments), 1 (up to 64: 4), 2 (8);
+//   bm = kBMFew (48): class 0 (up to 16 rows: 1 fragment), 1 (up to 32: 2), 2 (3).
+// Class c's tiles sit at tiles[c * cap ...] in group order, their count in ntiles[c].  A
+// 48-row tile also carries its row count (few_tile), one dependent read fewer at its start.
 constexpr int kBM = 128;
+constexpr int kBMFew = 48;
 constexpr int kTileClasses = 3;
 __host__ __device__ constexpr int class_fragments(int c) { return c == 0 ? 2 : c == 1 ? 4 : 8; }
+
+// A 48-row tile: group (9 bits), rows - 1 (6), first row (17; few_rows() bounds the rows).
+__host__ __device__ constexpr uint32_t few_tile(int e, int row0, int rows) {
+  return (uint32_t)e | (uint32_t)(rows - 1) << 9 | (uint32_t)row0 << 15;
+}
 
 // The tile table built by one workgroup of 64 * NW threads; thread e (e < ng) brings group
 // e's sorted rows [b, end).  The per-class bases are an exclusive prefix over the groups:
@@ -267,15 +274,16 @@ __host__ __device__ constexpr int class_fragments(int c) { return c == 0 ? 2 : c
 // of LDS).  Every thread of the workgroup calls it (it meets the workgroup once).
 template <int NW>
 __device__ __forceinline__ void tile_table_block(int e, int ng, int b, int end, uint32_t* __restrict__ tiles,
-                                                 int* __restrict__ ntiles, int cap, int (*wsum)[NW]) {
+                                                 int* __restrict__ ntiles, int cap, int bm, int (*wsum)[NW]) {
   const int lane = e & 63, wave = e >> 6;
   int full = 0, cnt[kTileClasses] = {0, 0, 0};
   if (e < ng) {
-    full = (end - b) / kBM;
-    const int rem = (end - b) % kBM;
-    cnt[2] = full + (rem > 64 ? 1 : 0);
-    cnt[1] = (rem > 32 && rem <= 64) ? 1 : 0;
-    cnt[0] = (rem > 0 && rem <= 32) ? 1 : 0;
+    const int c0 = bm == kBM ? 32 : 16, c1 = bm == kBM ? 64 : 32;  // most rows of classes 0 and 1
+    full = (end - b) / bm;
+    const int rem = (end - b) % bm;
+    cnt[2] = full + (rem > c1 ? 1 : 0);
+    cnt[1] = (rem > c0 && rem <= c1) ? 1 : 0;
+    cnt[0] = (rem > 0 && rem <= c0) ? 1 : 0;
   }
   int incl[kTileClasses];
 #pragma unroll
@@ -303,13 +311,16 @@ __device__ __forceinline__ void tile_table_block(int e, int ng, int b, int end, 
     base[c] = before + incl[c] - cnt[c];
     total[c] = all;
   }
+  auto entry = [&](int row) {
+    return bm == kBM ? (uint32_t)e | ((uint32_t)row << 9) : few_tile(e, row, min(bm, end - row));
+  };
   for (int i = 0; i < cnt[2]; ++i) {
     const int slot = base[2] + i;
-    if (slot < cap) tiles[2 * cap + slot] = (uint32_t)e | ((uint32_t)(b + i * kBM) << 9);
+    if (slot < cap) tiles[2 * cap + slot] = entry(b + i * bm);
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c)
-    if (cnt[c] && base[c] < cap) tiles[c * cap + base[c]] = (uint32_t)e | ((uint32_t)(b + full * kBM) << 9);
+    if (cnt[c] && base[c] < cap) tiles[c * cap + base[c]] = entry(b + full * bm);
   if (e < kTileClasses) ntiles[e] = min(e == 0 ? total[0] : e == 1 ? total[1] : total[2], cap);
 }
 
@@ -450,11 +461,12 @@ constexpr int kDispatchChunk = 1024;
 // With counted, counts[][] already hold the chunk counts (the prefill top-k adds them) and
 // the count kernel is skipped.
 // With tiles != nullptr the first scatter workgroup also writes the grouped GEMM's tile
-// table for the routed groups plus, when shared_rows > 0, a shared group of that many rows
+// table (tiles of bm rows) for the routed groups plus, when shared_rows > 0, a shared group of that many rows
 // (n_experts + 1 <= 256 groups then).
 hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int32_t* order, int32_t* inv,
                            int32_t* offsets, RmoeScratch& s, hipStream_t st, uint32_t* tiles = nullptr,
-                           int* ntiles = nullptr, int cap = 0, int shared_rows = 0, bool counted = false);
+                           int* ntiles = nullptr, int cap = 0, int shared_rows = 0, bool counted = false,
+                           int bm = kBM);
 
 // Prefill MoE (moe_prefill.hip).  With ids_in == nullptr the router runs on the device
 // and writes ids_out/wts_out; otherwise ids_in/wts_in are used.  With shared_gu the

@@ -1,0 +1,88 @@
+"""GPU: the grouped GEMM for groups of few rows (csrc/few_rows_gemm.h) against the general one.
+
+Both kernels take a row's products in the same order, so a token's output is the same bytes
+in a batch of few rows per expert and in one of many.  The batches put groups on both sides
+of the 16-, 32- and 48-row tile edges; I = 320 leaves half of the last gate/up tile and of
+the last down K tile empty; some token rows are scaled so that their h chunks carry
+different exponents."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from raon_npu_amd import geometry as G
+
+from moe_fixtures import make_layer, random_tokens
+from oracle import bfp16 as B
+
+pytestmark = pytest.mark.gpu
+
+GEOM = dict(hidden=512, inter=320, n_routed=16, n_shared=1, top_k=2)
+FEW, MANY = 200, 1200  # 25 and 150 rows per expert: below and above the line at 46
+
+
+def _routes(rng, T):
+    """Skewed routing: expert e is drawn ~ 1 / (1 + e), so group sizes span the tile edges."""
+    p = 1.0 / (1.0 + np.arange(16))
+    return np.stack([rng.choice(16, 2, replace=False, p=p / p.sum()) for _ in range(T)]).astype(np.int32)
+
+
+def _tokens(T, seed):
+    x = random_tokens(T, 512, seed)
+    u = x.astype(np.uint32)
+    # rows 5, 25, 45, ...: a hundred times 2^12 larger, rows 6, 26, ... 2^-14 smaller
+    for r0, shift in ((5, 12), (6, -14)):
+        e = (u[r0::20] >> 7) & 0xFF
+        u[r0::20] = (u[r0::20] & ~np.uint32(0xFF << 7)) | (np.clip(e.astype(np.int64) + shift, 1, 250).astype(np.uint32) << 7)
+    return u.astype(np.uint16)
+
+
+@pytest.mark.parametrize("layout", ["q4nx", "weights-d"])
+@pytest.mark.parametrize("betas", [(None, None), (4.0, 25.0)])
+def test_few_rows_equals_many_rows(gpu_ctx, layout, betas):
+    geom = G.MoeGeometry(**GEOM)
+    syn = make_layer(geom, seed=71)
+    rng = np.random.default_rng(72)
+    if layout == "q4nx":
+        lyr = gpu_ctx.create_layer(1700, geom)
+        lyr.upload_experts(syn.gate_up, syn.down)
+    else:
+        lyr = gpu_ctx.create_layer_d(1700, geom)
+        lyr.upload_d(1, 0, syn.gate_up[: geom.n_routed * geom.gu_bytes])
+        w = rng.normal(0.0, 0.02, (geom.n_experts, geom.hidden, geom.inter_pad)).astype(np.float32)
+        lyr.upload_d(2, 0, b"".join(B.pack_gemv(m) for m in w))
+    x, ids = _tokens(MANY, 73), _routes(rng, MANY)
+    wts = rng.uniform(0.1, 0.9, ids.shape).astype(np.float32)
+    sgu = random_tokens(MANY, 2 * geom.inter, 74)
+    want_r, want_s = lyr.moe_experts_grouped(x, ids, wts, sgu, *betas)
+    assert len(set(np.bincount(ids[:FEW].reshape(-1), minlength=16) // 16)) > 2  # several tile classes
+    for T in (1, 2, 17, 33, 48, 49, FEW):
+        r, s = lyr.moe_experts_grouped(x[:T], ids[:T], wts[:T], sgu[:T], *betas)
+        np.testing.assert_array_equal(r, want_r[:T], err_msg=f"routed, T={T}")
+        np.testing.assert_array_equal(s, want_s[:T], err_msg=f"shared, T={T}")
+    lyr.free()
+
+
+def test_few_rows_prefill_equals_many_rows(gpu_ctx):
+    """The device-routed form (the shared expert's gate/up in the layer) over the same line."""
+    import torch
+
+    geom = G.MoeGeometry(**GEOM)
+    syn = make_layer(geom, seed=75)
+    lyr = gpu_ctx.create_layer(1701, geom)
+    lyr.upload_experts(syn.gate_up, syn.down)
+    lyr.set_router(syn.router, score="softmax")
+    lyr.reserve(MANY)
+    x = torch.from_numpy(_tokens(MANY, 76).view(np.int16)).cuda()
+
+    def run(T):
+        out = torch.empty(T, geom.hidden, dtype=torch.int16, device="cuda")
+        lyr.moe_prefill_dev(x[:T].contiguous(), T, out, stream=torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    want = run(MANY)
+    for T in (1, 16, 47, FEW):
+        np.testing.assert_array_equal(run(T), want[:T], err_msg=f"T={T}")
+    lyr.free()

@@ -220,7 +220,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
               acc[m][f] = mfma16(b.s[m][2 - p / 2], (p & 1) ? bsc8 : bmin, acc[m][f]);
         }
       };
-      if constexpr (MF <= 2) {
+      if constexpr (MF <= 1) {
         CBlk ca, cb;
         load_blk(0, ca);
 #pragma unroll 1
@@ -234,7 +234,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
             corr_blk(blk + 1, cb);
           }
         }
-      } else {  // registers for one block
+      } else {  // registers for one block: two would spill, which has corrupted row addresses here
 #pragma unroll 1
         for (int blk = 0; blk < nblk; ++blk) {
           CBlk c;

@@ -8,7 +8,7 @@
 // places its assignments: its 4 waves take 256 consecutive assignments each, rank lanes
 // of equal expert with ballots (64 at a time, in order) and offset by the counts of the
 // waves before, so the sort is stable without atomics on the output.
-#include "rmoe_internal.h"
+#include "dispatch_block.h"
 
 namespace rmoe {
 namespace {
@@ -18,24 +18,7 @@ constexpr int kChunk = kDispatchChunk;
 __global__ __launch_bounds__(256) void dispatch_count_kernel(const int32_t* __restrict__ ids, int n, int E,
                                                              int32_t* __restrict__ counts, int* err) {
   __shared__ int hist[256];
-  const int c = blockIdx.x;
-  hist[threadIdx.x] = 0;
-  __syncthreads();
-  const int begin = c * kChunk;
-  int ev[kChunk / 256];
-#pragma unroll
-  for (int j = 0; j < kChunk / 256; ++j) {
-    const int i = begin + 256 * j + threadIdx.x;
-    ev[j] = i < n ? ids[i] : 0x7fffffff;
-  }
-#pragma unroll
-  for (int j = 0; j < kChunk / 256; ++j) {
-    if (ev[j] == 0x7fffffff) continue;
-    if (ev[j] >= 0 && ev[j] < E) atomicAdd(&hist[ev[j]], 1);
-    else atomicOr(err, 4);
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < E) counts[(size_t)c * E + threadIdx.x] = hist[threadIdx.x];
+  dispatch_count_block(ids, n, E, counts, err, blockIdx.x, hist);
 }
 
 // counts[c][e]: assignments of chunk c routed to expert e.  Workgroup c also writes

@@ -19,7 +19,7 @@
 #include <algorithm>
 
 #include "../../include/raon_moe.h"
-#include "rmoe_internal.h"
+#include "dispatch_block.h"
 #include "wave_gemm.h"
 
 namespace rmoe {
@@ -409,11 +409,6 @@ __device__ __forceinline__ void prep_x_block(const uint16_t* __restrict__ x, int
   }
   if (lane == 0) xe[t] = (int8_t)e;
 }
-__global__ __launch_bounds__(256) void prep_x_kernel(const uint16_t* __restrict__ x, int T, int K,
-                                                     uint16_t* __restrict__ xh, int8_t* __restrict__ xe,
-                                                     uint16_t* __restrict__ xsum) {
-  prep_x_block(x, T, K, xh, xe, xsum, blockIdx.x);
-}
 // The router GEMM and the activation-row preparation (both read only x) in one launch:
 // workgroups 0..n_router-1 are router workgroups (token block, K quarter, expert group),
 // the rest prepare four rows each.  One launch fewer on the routing's critical path.
@@ -464,7 +459,7 @@ struct GemmArgs {
   int inter;         // gate/up: I (the up rows start at I)
   int mode;          // 0: gate/up + activation -> h; 1: down -> D
   int n_tiles;       // WG N-tiles (gate/up: ceil(I/128) units of 128; down: N_total/256 rows of 256)
-  // activation rows (fp16 operands, see prep_x_kernel and the gate/up epilogue)
+  // activation rows (fp16 operands, see prep_x_block and the gate/up epilogue)
   const uint16_t* src;      // mode 0: xh [T, K] gathered by token; mode 1: h [rows, K] in sorted order
   const int8_t* aexp;       // power-of-two exponent of each src row (int8 [rows])
   const int32_t* order;     // mode 0: sorted position -> assignment (token*k + route)
@@ -495,6 +490,20 @@ struct GemmArgs {
 
 __device__ __forceinline__ int group_end(const GemmArgs& a, int e) {
   return e < a.n_routed ? a.offsets[e + 1] : a.shared_base + a.shared_rows;
+}
+
+// The padding of one h row past I: columns [I, Ipad), their group sums and the exponents of
+// the chunks past the last live one, all zero (they feed the zero-padded down columns).
+// The gate/up GEMM's last n-tile writes it, `n` lanes of a row taking pieces i, i + n, ...
+// (a launch of its own before the GEMM cost 5.4 us at 32 tokens; here nothing measurable).
+__device__ __forceinline__ void zero_row_padding(const GemmArgs& a, int row, int i, int n) {
+  uint64_t* h = reinterpret_cast<uint64_t*>(a.out + (size_t)row * a.out_ld);  // I % 64 == 0
+  for (int c = a.inter / 4 + i; c < a.out_ld / 4; c += n) h[c] = 0ull;
+  const int Gp = sum_planes_gp(a.out_ld / 32);
+  uint16_t* d = a.out_ssum + (size_t)row * 3 * Gp;
+  for (int g = a.inter / 32 + i; g < Gp; g += n) d[g] = d[Gp + g] = d[2 * Gp + g] = 0;
+  const int es = exp_stride(a.out_ld);
+  for (int c = (a.inter + 127) / 128 + i; c < a.out_ld / 128; c += n) a.out_exp[(size_t)row * es + c] = 0;
 }
 
 // A shared tile in a GEMM without shared rows (gate/up with the shared gate/up given).
@@ -1074,6 +1083,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const uint32_t* __r
                        bf16x2_to_f16x2(v.w, ex));
       if (r < nrows && c == 0) a.out_exp[(size_t)(row0 + r) * eso + nt] = (int8_t)ex;
     }
+    if (nt == a.n_tiles - 1)
+      for (int r = tid >> 4; r < nrows; r += 32) zero_row_padding(a, row0 + r, tid & 15, 16);
   } else {
     // Output columns 0..127 of the 256 in slot 0 (fragment 0), 128..255 in slot 1.
     // (bf16 by the hardware conversion: a NaN may keep its payload here; the combine
@@ -1330,7 +1341,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // A route whose expert id is outside [0, E) (device ids are not checked on the host; the
 // dispatch flags them with error bit 4 and places no row for them) adds nothing, so the
 // output does not depend on stale scratch before the error is reported.
-__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ D, int H, const int32_t* __restrict__ ids,
+// A small batch is bound by its chain of dependent loads, not by its bytes: one load round
+// for the routes and one pass of H / 8 threads over the columns (256 threads took two passes
+// at H = 2560) brought 32 tokens x 6 routes from 9.3 to 6.0 us, 6,700 x 6 stays at 53.5 us
+// (4.5 TB/s).
+__global__ __launch_bounds__(1024) void combine_kernel(const uint16_t* __restrict__ D, int H, const int32_t* __restrict__ ids,
                                                       const float* __restrict__ wts, const int32_t* __restrict__ inv,
                                                       int k, int E, int shared_base, const uint16_t* __restrict__ x,
                                                       uint16_t* __restrict__ out, uint16_t* __restrict__ routed,
@@ -1338,17 +1353,26 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   const int t = blockIdx.x;
   __shared__ int s_pos[16];
   __shared__ float s_w[16];
-  // Route q goes to slot rank(q) = its place in ascending expert order.
-  if ((int)threadIdx.x < k) {
-    const int q = threadIdx.x, eq = ids[(size_t)t * k + q];
+  // Route q goes to slot rank(q) = its place in ascending expert order: lane q of the first
+  // wave holds route q, and the ranks come from shuffles (one round of loads).
+  if (threadIdx.x < 64) {
+    const int q = threadIdx.x;
+    int eq = 0x7fffffff, pos = -1;
+    float wq = 0.f;
+    if (q < k) {
+      eq = ids[(size_t)t * k + q];
+      pos = inv[(size_t)t * k + q];
+      wq = wts[(size_t)t * k + q];
+    }
     int rank = 0;
     for (int q2 = 0; q2 < k; ++q2) {
-      const int e2 = ids[(size_t)t * k + q2];
+      const int e2 = __shfl(eq, q2, 64);
       rank += (e2 < eq) || (e2 == eq && q2 < q);
     }
-    const bool valid = eq >= 0 && eq < E;
-    s_pos[rank] = valid ? inv[(size_t)t * k + q] : -1;
-    s_w[rank] = wts[(size_t)t * k + q];
+    if (q < k) {
+      s_pos[rank] = eq >= 0 && eq < E ? pos : -1;
+      s_w[rank] = wq;
+    }
   }
   __syncthreads();
   // 8 columns (16 bytes) per thread per pass.
@@ -1407,34 +1431,16 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   }
 }
 
-// One wave per row: the h columns past I are zeroed, with the group sums of the groups
-// past I (and the planes' padding) and the chunk exponents past the last live chunk.
-__global__ __launch_bounds__(256) void zero_pad_cols_kernel(uint16_t* __restrict__ h, uint16_t* __restrict__ hsum,
-                                                            int8_t* __restrict__ hexp, int rows, int I, int Ipad) {
-  const size_t r = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  if (r >= (size_t)rows) return;
-  // I % 64 == 0: 4-column pieces of 8 bytes stay aligned.
-  for (int c = I + 4 * lane; c < Ipad; c += 256) *reinterpret_cast<uint64_t*>(h + r * Ipad + c) = 0ull;
-  // Groups entirely past I; a group straddling I gets its sum from the GEMM epilogue only
-  // when I is a multiple of 32 (guaranteed: I % 64 == 0).
-  const int Gp = sum_planes_gp(Ipad / 32);
-  uint16_t* d = hsum + r * 3 * Gp;
-  for (int g = I / 32 + lane; g < Gp; g += 64) d[g] = d[Gp + g] = d[2 * Gp + g] = 0;
-  const int es = exp_stride(Ipad);
-  for (int c = (I + 127) / 128 + lane; c < es; c += 64) hexp[r * es + c] = 0;
-}
-
 // h rows of the shared expert from a given shared_gu [T, 2I] (gate then up):
 // RTNE(act(g, u)) as the gate/up epilogue writes them (fp16 operand with one exponent
 // per 128-unit chunk, planar group sums, zero past I).  One wave per (token, chunk):
 // lane L takes columns 2L, 2L+1 of the chunk; a group's 32 columns are 16 lanes, summed
 // by shuffles.
-__global__ __launch_bounds__(256) void shared_act_kernel(const uint16_t* __restrict__ gu, int T, int I, int Ipad,
-                                                         int act, float gb, float vb, uint16_t* __restrict__ h,
-                                                         uint16_t* __restrict__ hsum, int8_t* __restrict__ hexp) {
+__device__ __forceinline__ void shared_act_block(const uint16_t* __restrict__ gu, int T, int I, int Ipad, int act,
+                                                 float gb, float vb, uint16_t* __restrict__ h,
+                                                 uint16_t* __restrict__ hsum, int8_t* __restrict__ hexp, int bx) {
   const int nch = Ipad / 128, Gp = sum_planes_gp(Ipad / 32), es = exp_stride(Ipad);
-  const size_t wid = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const size_t wid = (size_t)bx * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (wid >= (size_t)T * nch) return;
   const int t = (int)(wid / nch), ch = (int)(wid % nch);
@@ -1462,8 +1468,35 @@ __global__ __launch_bounds__(256) void shared_act_kernel(const uint16_t* __restr
     for (int c = nch + lane; c < es; c += 64) hexp[(size_t)t * es + c] = 0;
 }
 
+// What a grouped call with its routing given needs before the dispatch's scatter, in one
+// launch: workgroups 0..n_x-1 prepare four activation rows each, the next n_cnt count a
+// dispatch chunk each, the rest compute four (token, chunk) pieces of the shared h rows.
+// Each part alone is a launch of about 5 us whatever its size below some hundred tokens:
+// 256 tokens at H = 2560, I = 1088 took 6.6 + 4.7 + 5.5 us in three launches, 7.6 in this one.
+struct GroupedPrepArgs {
+  const uint16_t *x, *gu;
+  int T, K, I, Ipad, n_x, n_cnt, n, E, act;
+  float gb, vb;
+  const int32_t* ids;
+  int32_t* counts;
+  int* err;
+  uint16_t *xh, *xsum, *h, *hsum;
+  int8_t *xe, *hexp;
+};
+__global__ __launch_bounds__(256) void grouped_prep_kernel(GroupedPrepArgs a) {
+  __shared__ int hist[256];
+  int b = blockIdx.x;
+  if (b < a.n_x) {
+    prep_x_block(a.x, a.T, a.K, a.xh, a.xe, a.xsum, b);
+  } else if ((b -= a.n_x) < a.n_cnt) {
+    dispatch_count_block(a.ids, a.n, a.E, a.counts, a.err, b, hist);
+  } else {
+    shared_act_block(a.gu, a.T, a.I, a.Ipad, a.act, a.gb, a.vb, a.h, a.hsum, a.hexp, b - a.n_cnt);
+  }
+}
+
 // One exponent per h row for the down GEMM: the row's chunks (128 units, one exponent
-// each from the gate/up epilogue or shared_act_kernel) are brought to the largest chunk
+// each from the gate/up epilogue or shared_act_block) are brought to the largest chunk
 // exponent; a chunk below it is rescaled by 2^(e_c - e_row) (values more than 2^38
 // below the row's largest keep their fp16 grid rounding).  Rows whose chunks agree,
 // nearly all, only read their exponents.  Thread per row.
@@ -1638,38 +1671,52 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   hipError_t err;
   const int32_t* ids = ids_in;
   const float* wts = wts_in;
-  // With the routing on the device, the router GEMM launch also prepares the activation
-  // rows and clears the dispatch chunk counts, which the top-k then adds up (no count
-  // kernel).
-  const int nchunks = (int)((A + kDispatchChunk - 1) / kDispatchChunk);
-  const bool counted = !ids_in && (size_t)nchunks * E <= s.chunk_elems;
-  if (!ids_in) {
-    err = launch_router_prep(x, T, L.H, L.router_w, E, logits, xh, xexp, xsum, counted ? s.chunk_counts : nullptr,
-                             counted ? nchunks * E : 0, st);
-    if (err != hipSuccess) return err;
-    err = launch_topk(logits, T, E, k, L.score, L.router_bias, L.renorm, L.scaling, ids_out, wts_out,
-                      counted ? s.chunk_counts : nullptr, st);
-    if (err != hipSuccess) return err;
-    ids = ids_out;
-    wts = wts_out;
-  } else {
-    hipLaunchKernelGGL(prep_x_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, x, T, L.H, xh, xexp, xsum);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
-  }
   // One tile table for both GEMMs: the routed groups and the shared one, whose tiles the
   // gate/up GEMM skips when its gate/up is given.
   const bool fused_table = E + 1 <= 256;
-  err = fused_table ? launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, tiles, ntiles, tile_cap, T,
-                                      counted, bm)
-                    : launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, nullptr, nullptr, 0, 0, counted);
-  if (err != hipSuccess) return err;
-  if (L.Ipad > L.I) {
-    // h columns past I (their group sums and chunk exponents) feed the zero-padded down
-    // columns.
-    hipLaunchKernelGGL(zero_pad_cols_kernel, dim3((unsigned)((R + 3) / 4)), dim3(256), 0, st, h, hsum, hexp,
-                       (int)R, L.I, L.Ipad);
+  const int nchunks = (int)((A + kDispatchChunk - 1) / kDispatchChunk);
+  if (!ids_in) {
+    // The router GEMM launch also prepares the activation rows and clears the dispatch chunk
+    // counts, which the top-k then adds up (no count kernel).
+    if ((err = launch_router_prep(x, T, L.H, L.router_w, E, logits, xh, xexp, xsum, s.chunk_counts, nchunks * E, st)) !=
+        hipSuccess)
+      return err;
+    if ((err = launch_topk(logits, T, E, k, L.score, L.router_bias, L.renorm, L.scaling, ids_out, wts_out,
+                           s.chunk_counts, st)) != hipSuccess)
+      return err;
+    ids = ids_out;
+    wts = wts_out;
+  } else {
+    GroupedPrepArgs p{};
+    p.x = x;
+    p.gu = shared_gu;
+    p.T = T;
+    p.K = L.H;
+    p.I = L.I;
+    p.Ipad = L.Ipad;
+    p.n_x = (T + 3) / 4;
+    p.n_cnt = nchunks;
+    p.n = (int)A;
+    p.E = E;
+    p.act = act;
+    p.gb = gb;
+    p.vb = vb;
+    p.ids = ids_in;
+    p.counts = s.chunk_counts;
+    p.err = s.err;
+    p.xh = xh;
+    p.xsum = xsum;
+    p.xe = xexp;
+    p.h = h + A * L.Ipad;
+    p.hsum = hsum + A * 3 * Gph;
+    p.hexp = hexp + A * exp_stride(L.Ipad);
+    const size_t n_act = shared_gu ? ((size_t)T * (L.Ipad / 128) + 3) / 4 : 0;
+    hipLaunchKernelGGL(grouped_prep_kernel, dim3((unsigned)(p.n_x + p.n_cnt + n_act)), dim3(256), 0, st, p);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
+  err = fused_table ? launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, tiles, ntiles, tile_cap, T, true, bm)
+                    : launch_dispatch(ids, T, k, E, s.order, s.inv, s.offsets, s, st, nullptr, nullptr, 0, 0, true);
+  if (err != hipSuccess) return err;
   // Gate/up (+ activation): routed groups, and the shared expert unless its gate/up is given.
   GemmArgs g{};
   g.wbase = L.gu;
@@ -1702,12 +1749,6 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
                        tile_cap, bm);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
-  if (shared_gu) {
-    const size_t n = (size_t)T * (L.Ipad / 128);  // waves, 4 per block
-    hipLaunchKernelGGL(shared_act_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, shared_gu, T, L.I,
-                       L.Ipad, act, gb, vb, h + A * L.Ipad, hsum + A * 3 * Gph, hexp + A * exp_stride(L.Ipad));
-    if ((err = hipGetLastError()) != hipSuccess) return err;
-  }
   if ((err = launch_grouped(g, tiles, ntiles, tile_cap, E, st, false, few)) != hipSuccess) return err;
   if (!few) {  // few_rows_tile takes the chunks' exponents itself
     hipLaunchKernelGGL(h_unify_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, h, hexp, (int)R, L.Ipad,
@@ -1737,7 +1778,9 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   // more of D in the caches.
   d.out_nt = R * (size_t)L.H * 2 > ((size_t)64 << 20) ? 1 : 0;
   if ((err = launch_grouped(d, tiles, ntiles, tile_cap, E, st, L.dn_fmt == RMOE_FMT_BFP16, few)) != hipSuccess) return err;
-  hipLaunchKernelGGL(combine_kernel, dim3(T), dim3(256), 0, st, D, L.H, ids, wts, s.inv, k, E, (int)A,
+  // One pass of 8 columns per thread (H = 2560: 320 threads), up to 8192 columns.
+  const int cthreads = std::min(1024, (L.H / 8 + 63) / 64 * 64);
+  hipLaunchKernelGGL(combine_kernel, dim3(T), dim3(cthreads), 0, st, D, L.H, ids, wts, s.inv, k, E, (int)A,
                      residual ? x : nullptr, out, routed, shared_down, 1);
   return hipGetLastError();
 }

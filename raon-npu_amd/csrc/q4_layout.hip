@@ -65,38 +65,67 @@ __global__ void relayout_in_kernel(const uint8_t* __restrict__ packed, uint8_t* 
   *reinterpret_cast<uint32_t*>(t + kCodeBytes + lane * 16 + j * 4) = scale | (mn << 16);
 }
 
-// Thread = (row pair, group): writes both rows' nibbles (one byte per column).
-__global__ void relayout_out_kernel(const uint8_t* __restrict__ tiles, uint8_t* __restrict__ packed, int M, int K) {
-  const int G = K / 32, nkt = K / 128;
-  const size_t n = (size_t)(M / 2) * G;
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int g = (int)(idx % G);
-  const int r0 = (int)(idx / G) * 2;
-  const int kt = g / 4, j = g % 4;
-  uint32_t w[2][4];
-  uint32_t smv[2];
+// One workgroup per 64 rows x 256 columns: two K tiles, 10 KB in a row in the tile layout,
+// become two pack_gemv blocks, 10 KB in a row there, through LDS, so that both sides move
+// 16 bytes per lane.  (One thread per row pair and group, storing 32 single bytes 8 apart,
+// took 16.4 us for 1536 x 2048; this takes 5.3 us.)  A group's 1 KB of codes is followed by
+// 16 bytes of padding in LDS: the lanes of a wave read one row of four groups at a time.
+constexpr int kRelayoutGroup = 1024 + 16;  // bytes per group of 64 rows in LDS
+__global__ __launch_bounds__(256) void relayout_out_kernel(const uint8_t* __restrict__ tiles,
+                                                           uint8_t* __restrict__ packed, int K) {
+  __shared__ __attribute__((aligned(16))) uint8_t codes[8 * kRelayoutGroup];
+  __shared__ __attribute__((aligned(16))) uint32_t sm[2][64 * 4];
+  const int kblocks = K / 256, tid = threadIdx.x;
+  const int band = blockIdx.x / kblocks, kb = blockIdx.x % kblocks;
+  const uint4* src = reinterpret_cast<const uint4*>(tiles + ((size_t)band * kblocks + kb) * 2 * kTileBytes);
+  constexpr int kUnits = kTileBytes / 16;  // 320: four groups of 64 rows, then the scale|min words
+  uint4 v[3];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = r0 + h;
-    const uint8_t* t = tiles + ((size_t)(r / 64) * nkt + kt) * kTileBytes;
-    const uint4 c = *reinterpret_cast<const uint4*>(t + j * 1024 + (r % 64) * 16);
-    w[h][0] = c.x; w[h][1] = c.y; w[h][2] = c.z; w[h][3] = c.w;
-    smv[h] = *reinterpret_cast<const uint32_t*>(t + kCodeBytes + (r % 64) * 16 + j * 4);
+  for (int i = 0; i < 3; ++i)
+    if (tid + 256 * i < 2 * kUnits) v[i] = src[tid + 256 * i];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int u = tid + 256 * i;
+    if (u >= 2 * kUnits) continue;
+    const int t = u / kUnits, o = u % kUnits;
+    if (o < 256) *reinterpret_cast<uint4*>(codes + (4 * t + (o >> 6)) * kRelayoutGroup + (o & 63) * 16) = v[i];
+    else *reinterpret_cast<uint4*>(&sm[t][(o - 256) * 4]) = v[i];
   }
-  const PackPos p = pack_pos(r0, g, K);
-  uint16_t* sm = reinterpret_cast<uint16_t*>(packed + p.base);
-  sm[p.gg * 32 + p.r32] = (uint16_t)(smv[0] & 0xffffu);
-  sm[p.gg * 32 + p.r32 + 1] = (uint16_t)(smv[1] & 0xffffu);
-  sm[256 + p.gg * 32 + p.r32] = (uint16_t)(smv[0] >> 16);
-  sm[256 + p.gg * 32 + p.r32 + 1] = (uint16_t)(smv[1] >> 16);
-  uint8_t* cbase = packed + p.base + 1024 + (size_t)((p.half * 8 + p.gg) * 32) * 8 + (p.r16 >> 1);
-#pragma unroll 8
-  for (int c = 0; c < 32; ++c) {
-    const int ni = tile_nibble_index(c);
-    const uint32_t lo = (w[0][ni >> 3] >> (4 * (ni & 7))) & 15u;
-    const uint32_t hi = (w[1][ni >> 3] >> (4 * (ni & 7))) & 15u;
-    cbase[c * 8] = (uint8_t)(lo | (hi << 4));
+  __syncthreads();
+  // Blocks 2 * (band % 2) and the next of the 128-row slice.
+  uint4* dst = reinterpret_cast<uint4*>(packed + (((size_t)(band >> 1) * kblocks + kb) * 4 + 2 * (band & 1)) * 5120);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int u = tid + 256 * i;
+    if (u >= 2 * kUnits) continue;
+    const int blk = u / kUnits, o = u % kUnits;
+    uint32_t w[4];
+    if (o < 64) {  // 8 rows' scales (units 0..31) or mins of one group
+      const int gg = (o & 31) >> 2, r0 = 32 * blk + 8 * (o & 3), hi = o >> 5;
+      const uint32_t* p = &sm[gg >> 2][r0 * 4 + (gg & 3)];
+      const uint32_t sel = hi ? 0x07060302u : 0x05040100u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) w[q] = __builtin_amdgcn_perm(p[8 * q + 4], p[8 * q], sel);
+    } else {  // columns 2 cp and 2 cp + 1 of one group, 16 rows: 8 bytes each, two rows per byte
+      const int q = o - 64, cp = q & 15, gg = (q >> 4) & 7, r0 = 32 * blk + 16 * (q >> 7);
+      const uint8_t* p = codes + gg * kRelayoutGroup + r0 * 16 + 4 * (cp >> 2);
+      const int sh = 4 * (cp & 3);  // nibbles cp % 4 (even column) and cp % 4 + 4 (odd column)
+      uint32_t b[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t lo = *reinterpret_cast<const uint32_t*>(p + 32 * j) >> sh;
+        const uint32_t hi = *reinterpret_cast<const uint32_t*>(p + 32 * j + 16) >> sh;
+        b[j] = (lo & 0x000f000fu) | ((hi & 0x000f000fu) << 4);  // bytes 0 and 2
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = 4 * (j & 1);  // even column: bytes 0 of b; odd column: bytes 2
+        const uint32_t sel = j < 2 ? 0x0c0c0400u : 0x0c0c0602u;
+        const uint32_t p0 = __builtin_amdgcn_perm(b[k + 1], b[k], sel), p1 = __builtin_amdgcn_perm(b[k + 3], b[k + 2], sel);
+        w[j] = p0 | (p1 << 16);
+      }
+    }
+    dst[u] = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 
@@ -236,19 +265,36 @@ __device__ __forceinline__ GroupIndex group_index(size_t idx, int nkt) {
   return gi;
 }
 
-__global__ void quantize_kernel(const float* __restrict__ w, int M, int K, int ld, int k_valid,
-                                uint8_t* __restrict__ tiles, int* __restrict__ err) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (size_t)M * (K / 32)) return;
-  const GroupIndex gi = group_index(idx, K / 128);
-  const float* row = w + (size_t)gi.r * ld;
+// One workgroup per tile of 64 rows x 128 columns, whose fp32 values come through LDS: a
+// wave loads its 16 rows by whole 256-byte lines, then takes group `wave` of row `lane`.
+// (A thread loading its own 128 bytes touched 64 lines per load: 15.4 us for 1536 x 2048;
+// this takes 9.7 us.  The rest is the serial fp64 divisions of 1.5 waves per SIMD.)
+constexpr int kQuantRow = 128 + 4;  // floats per row in LDS: 16-byte reads of 64 rows spread over the banks
+__global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__ w, int K, int ld, int k_valid,
+                                                       uint8_t* __restrict__ tiles, int* __restrict__ err) {
+  __shared__ __attribute__((aligned(16))) float rows[64 * kQuantRow];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int nkt = K / kTileCols, rt = blockIdx.x / nkt, kt = blockIdx.x % nkt;
+  const float* src = w + (size_t)(rt * 64 + 16 * wave) * ld + kt * kTileCols;
+  float x[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const int c = lane + 64 * (i & 1);
+    x[i] = kt * kTileCols + c < k_valid ? src[(size_t)(i >> 1) * ld + c] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < 32; ++i) rows[(16 * wave + (i >> 1)) * kQuantRow + lane + 64 * (i & 1)] = x[i];
+  __syncthreads();
   float v[32];
 #pragma unroll
-  for (int c = 0; c < 32; ++c) {
-    const int col = gi.g * 32 + c;
-    v[c] = col < k_valid ? row[col] : 0.f;
+  for (int c = 0; c < 32; c += 4) {
+    const float4 f = *reinterpret_cast<const float4*>(&rows[lane * kQuantRow + 32 * wave + c]);
+    v[c] = f.x;
+    v[c + 1] = f.y;
+    v[c + 2] = f.z;
+    v[c + 3] = f.w;
   }
-  quantize_group(v, tiles + gi.tile * kTileBytes, gi.j, gi.lane, err);
+  quantize_group(v, tiles + (size_t)blockIdx.x * kTileBytes, wave, lane, err);
 }
 
 // Counter-based N(0, std) weights: splitmix64 of (seed, row*k_valid + col) -> Box-Muller.
@@ -298,17 +344,17 @@ hipError_t launch_q4k_to_tiles(const uint8_t* q4k, int M, int K, uint8_t* tiles,
 }
 
 hipError_t launch_relayout_out(const uint8_t* tiles, uint8_t* packed, int M, int K, hipStream_t st) {
-  const size_t n = (size_t)(M / 2) * (K / 32);
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(relayout_out_kernel, dim3(blocks), dim3(256), 0, st, tiles, packed, M, K);
+  if (M % 64 || K % 256) return hipErrorInvalidValue;
+  const unsigned blocks = (unsigned)((M / 64) * (K / 256));
+  hipLaunchKernelGGL(relayout_out_kernel, dim3(blocks), dim3(256), 0, st, tiles, packed, K);
   return hipGetLastError();
 }
 
 hipError_t launch_quantize(const float* w, int M, int K, int ld, int k_valid, uint8_t* tiles, int* err,
                            hipStream_t st) {
-  const size_t n = (size_t)M * (K / 32);
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(quantize_kernel, dim3(blocks), dim3(256), 0, st, w, M, K, ld, k_valid, tiles, err);
+  if (M % 64 || K % kTileCols) return hipErrorInvalidValue;
+  const unsigned blocks = (unsigned)((M / 64) * (K / kTileCols));
+  hipLaunchKernelGGL(quantize_kernel, dim3(blocks), dim3(256), 0, st, w, K, ld, k_valid, tiles, err);
   return hipGetLastError();
 }
 

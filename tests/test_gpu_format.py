@@ -73,3 +73,22 @@ def test_expert_quantizer_pads_down_columns(gpu_ctx):
     assert got_gu == pack_gemv(*quantize(gu))
     assert got_dn == pack_gemv(*quantize(pad(dn, 128, 256)[0]))
     lyr.free()
+
+
+@pytest.mark.parametrize("M, K, offset", [(128, 256, 1), (384, 768, 3), (256, 2304, 0)])
+def test_quantize_and_download_tiles(gpu_ctx, M, K, offset):
+    """Tile and block edges of the LDS transposes; a source that is 4-byte aligned only."""
+    import torch
+
+    rng = np.random.default_rng(M + K)
+    w = rng.normal(0.0, 0.02, (M, K)).astype(np.float32)
+    buf = torch.zeros(M * K + 4, dtype=torch.float32, device="cuda")
+    buf[offset : offset + M * K] = torch.from_numpy(w).cuda().reshape(-1)
+    torch.cuda.synchronize()
+    mat = gpu_ctx.quantize_matrix(buf[offset : offset + M * K].view(M, K), M, K)
+    assert bytes(mat.download()) == pack_gemv(*quantize(w))
+    mat.free()
+    blob = rng.integers(0, 256, M * K * 5 // 8, dtype=np.uint8).tobytes()
+    mat = gpu_ctx.upload_matrix(blob, M, K)
+    assert bytes(mat.download()) == blob
+    mat.free()

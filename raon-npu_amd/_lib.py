@@ -128,6 +128,19 @@ def call(name: str, *args) -> None:
     check(getattr(load(), name)(*args))
 
 
+def new_bytes(n: int) -> tuple[bytes, int]:
+    """A bytes object of n bytes for the library to fill, and their address (filled before
+    anyone else sees the object; saves the copy out of a temporary array)."""
+    b = _new_bytes(None, n)
+    return b, _bytes_address(b)
+
+
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.argtypes, _new_bytes.restype = [_p, C.c_ssize_t], C.py_object
+_bytes_address = C.pythonapi.PyBytes_AsString
+_bytes_address.argtypes, _bytes_address.restype = [C.py_object], _p
+
+
 def ptr(a) -> int | None:
     """Raw pointer of a NumPy array or a torch tensor (None passes NULL)."""
     if a is None:

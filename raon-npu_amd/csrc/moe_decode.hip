@@ -417,7 +417,20 @@ __global__ __launch_bounds__(1024) void decode_down_band_kernel(DecodeArgs a0) {
   if (a.out) a.out[row] = (uint16_t)o;
 }
 
+__global__ __launch_bounds__(256) void copy16_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, unsigned n) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 }  // namespace
+
+hipError_t launch_copy16(const void* src, void* dst, size_t n, hipStream_t st) {
+  const unsigned units = (unsigned)(n / 16);
+  if (n % 16 || units == 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(copy16_kernel, dim3((units + 255) / 256), dim3(256), 0, st, static_cast<const uint4*>(src),
+                     static_cast<uint4*>(dst), units);
+  return hipGetLastError();
+}
 
 hipError_t launch_route(const RmoeLayer& L, const uint16_t* x, int T, int32_t* ids, float* wts, float* logits,
                         RmoeScratch& s, hipStream_t st) {

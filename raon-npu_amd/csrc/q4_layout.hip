@@ -72,11 +72,13 @@ __global__ void relayout_in_kernel(const uint8_t* __restrict__ packed, uint8_t* 
 // 16 bytes of padding in LDS: the lanes of a wave read one row of four groups at a time.
 constexpr int kRelayoutGroup = 1024 + 16;  // bytes per group of 64 rows in LDS
 __global__ __launch_bounds__(256) void relayout_out_kernel(const uint8_t* __restrict__ tiles,
-                                                           uint8_t* __restrict__ packed, int K) {
+                                                           uint8_t* __restrict__ packed, int K, unsigned first) {
   __shared__ __attribute__((aligned(16))) uint8_t codes[8 * kRelayoutGroup];
   __shared__ __attribute__((aligned(16))) uint32_t sm[2][64 * 4];
   const int kblocks = K / 256, tid = threadIdx.x;
-  const int band = blockIdx.x / kblocks, kb = blockIdx.x % kblocks;
+  // Workgroups in the order of the output: the two 64-row bands of a 128-row slice alternate.
+  const unsigned unit = first + blockIdx.x;
+  const int band = (int)(unit / (2 * kblocks)) * 2 + (int)(unit & 1), kb = (int)((unit >> 1) % kblocks);
   const uint4* src = reinterpret_cast<const uint4*>(tiles + ((size_t)band * kblocks + kb) * 2 * kTileBytes);
   constexpr int kUnits = kTileBytes / 16;  // 320: four groups of 64 rows, then the scale|min words
   uint4 v[3];
@@ -92,8 +94,7 @@ __global__ __launch_bounds__(256) void relayout_out_kernel(const uint8_t* __rest
     else *reinterpret_cast<uint4*>(&sm[t][(o - 256) * 4]) = v[i];
   }
   __syncthreads();
-  // Blocks 2 * (band % 2) and the next of the 128-row slice.
-  uint4* dst = reinterpret_cast<uint4*>(packed + (((size_t)(band >> 1) * kblocks + kb) * 4 + 2 * (band & 1)) * 5120);
+  uint4* dst = reinterpret_cast<uint4*>(packed + (size_t)blockIdx.x * kRelayoutBytes);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int u = tid + 256 * i;
@@ -343,10 +344,12 @@ hipError_t launch_q4k_to_tiles(const uint8_t* q4k, int M, int K, uint8_t* tiles,
   return hipGetLastError();
 }
 
-hipError_t launch_relayout_out(const uint8_t* tiles, uint8_t* packed, int M, int K, hipStream_t st) {
-  if (M % 64 || K % 256) return hipErrorInvalidValue;
-  const unsigned blocks = (unsigned)((M / 64) * (K / 256));
-  hipLaunchKernelGGL(relayout_out_kernel, dim3(blocks), dim3(256), 0, st, tiles, packed, K);
+hipError_t launch_relayout_out(const uint8_t* tiles, uint8_t* packed, int M, int K, size_t first, size_t n,
+                               hipStream_t st) {
+  const size_t total = (size_t)(M / 64) * (K / 256);
+  if (M % 128 || K % 256 || first >= total) return hipErrorInvalidValue;
+  const size_t count = n ? min(n, total - first) : total - first;
+  hipLaunchKernelGGL(relayout_out_kernel, dim3((unsigned)count), dim3(256), 0, st, tiles, packed, K, (unsigned)first);
   return hipGetLastError();
 }
 

@@ -78,6 +78,76 @@ int io_area(rmoe_ctx* ctx, size_t bytes, uint8_t** out) {
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// The context's pinned block: an input slot, an output slot, then the chunks of a download.
+// One token's routed experts took 57 us through three pageable copies in and one out, of
+// which 22 us are the kernels; 42 us this way.  Chunks of 512 KB: a transfer of about
+// 10 us, so the first one and the last host copy, which nothing overlaps, stay small (an
+// expert's 2.95 MB came down in 190 us, 111 this way; PCIe alone takes 57).
+constexpr size_t kPinnedIo = (size_t)256 << 10, kChunk = (size_t)512 << 10;
+constexpr int kChunks = 4;
+constexpr size_t kPinnedBytes = 2 * kPinnedIo + kChunks * kChunk;
+
+// One matrix of a download: tiles of an [M, K] matrix of format fmt to nbytes at host.
+struct Stretch {
+  const uint8_t* tiles;
+  int M, K, fmt;
+  uint8_t* host;
+  size_t nbytes;
+};
+// The chunk at `offset` of a stretch, n bytes, into pinned slot `slot` (queued).  q4nx: the
+// re-layout launch writes the slot itself.  bfp16: re-laid out into the staging buffer as a
+// whole with the first chunk, then copied.
+hipError_t fill_chunk(rmoe_ctx* ctx, const Stretch& p, int slot, size_t offset, size_t n) {
+  const size_t at = 2 * kPinnedIo + slot * kChunk;
+  if (p.fmt != RMOE_FMT_BFP16)
+    return rmoe::launch_relayout_out(p.tiles, ctx->pinned_dev + at, p.M, p.K, offset / rmoe::kRelayoutBytes,
+                                     n / rmoe::kRelayoutBytes, ctx->stream);
+  if (offset == 0) {
+    hipError_t e = rmoe::launch_b16_relayout_out(p.tiles, ctx->s.staging, p.M, p.K, ctx->stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipMemcpyAsync(ctx->pinned + at, ctx->s.staging + offset, n, hipMemcpyDeviceToHost, ctx->stream);
+}
+// Chunk after chunk through the pinned slots: the device fills up to kChunks ahead while the
+// host copies the oldest out.  (hipMemcpyAsync into pageable memory did the two in turn, and
+// waited for one matrix before it began the next.)
+int download_chunked(rmoe_ctx* ctx, const Stretch* parts, int n_parts) {
+  constexpr size_t kPer = kChunk / rmoe::kRelayoutBytes * rmoe::kRelayoutBytes;
+  for (int p = 0; p < n_parts; ++p)
+    if (parts[p].fmt == RMOE_FMT_BFP16) TRY(grow(ctx->s.staging, ctx->s.staging_bytes, parts[p].nbytes, ctx));
+  struct Cursor {
+    int part = 0;
+    size_t offset = 0, seq = 0;
+  } put, get;
+  auto advance = [&](Cursor& c) {
+    ++c.seq;
+    if ((c.offset += kPer) >= parts[c.part].nbytes) {
+      ++c.part;
+      c.offset = 0;
+    }
+  };
+  auto len = [&](const Cursor& c) { return std::min(kPer, parts[c.part].nbytes - c.offset); };
+  hipError_t e = hipSuccess;
+  while (e == hipSuccess && get.part < n_parts) {
+    while (e == hipSuccess && put.part < n_parts && put.seq < get.seq + kChunks) {
+      const int slot = (int)(put.seq % kChunks);
+      if ((e = fill_chunk(ctx, parts[put.part], slot, put.offset, len(put))) == hipSuccess)
+        e = hipEventRecord(ctx->chunk_done[slot], ctx->stream);
+      advance(put);
+    }
+    const int slot = (int)(get.seq % kChunks);
+    if (e == hipSuccess && (e = hipEventSynchronize(ctx->chunk_done[slot])) == hipSuccess) {
+      memcpy(parts[get.part].host + get.offset, ctx->pinned + 2 * kPinnedIo + slot * kChunk, len(get));
+      advance(get);
+    }
+  }
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(ctx->stream);  // nothing queued here may still write the slots
+    return fail(RMOE_EDEVICE, "download: %s", hipGetErrorString(e));
+  }
+  return RMOE_OK;
+}
+
 int check_layer(rmoe_ctx* ctx, int layer, RmoeLayer** out) {
   if (!ctx) return fail(RMOE_EINVAL, "null context");
   auto it = ctx->layers.find(layer);
@@ -269,6 +339,16 @@ uint8_t* static_scratch(int device) {
 
 }  // namespace
 
+// What rmoe_create sets up: the stream, the error word, the pinned block.  Deletes ctx.
+static void free_base(rmoe_ctx* ctx) {
+  for (hipEvent_t ev : ctx->chunk_done)
+    if (ev) (void)hipEventDestroy(ev);
+  if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+  hipFree(ctx->s.err);
+  hipStreamDestroy(ctx->stream);
+  delete ctx;
+}
+
 extern "C" {
 
 const char* rmoe_last_error(void) { return g_err.c_str(); }
@@ -296,10 +376,15 @@ int rmoe_create(int device, rmoe_ctx** out) {
   hipStreamSynchronize(ctx->stream);
   if (init_static_scratch(ctx) != RMOE_OK) {
     const std::string msg = g_err;
-    hipFree(ctx->s.err);
-    hipStreamDestroy(ctx->stream);
-    delete ctx;
+    free_base(ctx);
     return fail(RMOE_EDEVICE, "%s", msg.c_str());
+  }
+  bool ok = hipHostMalloc((void**)&ctx->pinned, kPinnedBytes, hipHostMallocDefault) == hipSuccess &&
+            hipHostGetDevicePointer((void**)&ctx->pinned_dev, ctx->pinned, 0) == hipSuccess;
+  for (hipEvent_t& ev : ctx->chunk_done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+  if (!ok) {
+    free_base(ctx);
+    return fail(RMOE_ENOMEM, "%zu bytes of pinned host memory failed", kPinnedBytes);
   }
   // The persistent decode kernel runs one workgroup per CU and needs all of them
   // resident at once.
@@ -326,7 +411,7 @@ int rmoe_destroy(rmoe_ctx* ctx) {
   }
   RmoeScratch& s = ctx->s;
   void* bufs[] = {s.part, s.counters, s.h, s.ids, s.wts, s.logits, s.order, s.inv, s.offsets,
-                  s.chunk_counts, s.err, s.staging, s.pf, s.stack, s.stack_cnt};
+                  s.chunk_counts, s.staging, s.pf, s.stack, s.stack_cnt};
   for (void* b : bufs)
     if (b) hipFree(b);
   auto it = g_io.find(ctx);
@@ -334,8 +419,7 @@ int rmoe_destroy(rmoe_ctx* ctx) {
     hipFree(it->second.p);
     g_io.erase(it);
   }
-  hipStreamDestroy(ctx->stream);
-  delete ctx;
+  free_base(ctx);
   return RMOE_OK;
 }
 
@@ -461,14 +545,8 @@ int rmoe_matrix_download(rmoe_ctx* ctx, int handle, void* bytes, size_t nbytes) 
   const size_t need = stored_bytes(*m);
   if (!bytes || nbytes != need) return fail(RMOE_EINVAL, "download buffer must hold %zu bytes", need);
   HIP_TRY(hipSetDevice(ctx->device));
-  TRY(grow(ctx->s.staging, ctx->s.staging_bytes, need, ctx));
-  if (m->fmt == RMOE_FMT_BFP16)
-    HIP_TRY(rmoe::launch_b16_relayout_out(m->tiles, ctx->s.staging, m->M, m->K, ctx->stream));
-  else
-    HIP_TRY(rmoe::launch_relayout_out(m->tiles, ctx->s.staging, m->M, m->K, ctx->stream));
-  HIP_TRY(hipMemcpyAsync(bytes, ctx->s.staging, need, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
-  return RMOE_OK;
+  const Stretch part{m->tiles, m->M, m->K, m->fmt, static_cast<uint8_t*>(bytes), need};
+  return download_chunked(ctx, &part, 1);
 }
 
 int rmoe_matrix_free(rmoe_ctx* ctx, int handle) {
@@ -788,19 +866,11 @@ int rmoe_layer_download_expert(rmoe_ctx* ctx, int layer, int expert, void* gate_
   if ((has_gu ? (!gate_up || gu_nbytes != L->gu_bytes) : (gate_up != nullptr)) || !down || dn_nbytes != L->dn_bytes)
     return fail(RMOE_EINVAL, "download buffers must hold %zu and %zu bytes", has_gu ? L->gu_bytes : 0, L->dn_bytes);
   HIP_TRY(hipSetDevice(ctx->device));
-  TRY(grow(ctx->s.staging, ctx->s.staging_bytes, std::max(L->gu_bytes, L->dn_bytes), ctx));
-  if (has_gu) {
-    HIP_TRY(rmoe::launch_relayout_out(L->gu + (size_t)expert * L->gu_bytes, ctx->s.staging, 2 * L->I, L->H, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(gate_up, ctx->s.staging, L->gu_bytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-  }
-  if (L->dn_fmt == RMOE_FMT_BFP16)
-    HIP_TRY(rmoe::launch_b16_relayout_out(L->dn + (size_t)expert * L->dn_bytes, ctx->s.staging, L->H, L->Ipad, ctx->stream));
-  else
-    HIP_TRY(rmoe::launch_relayout_out(L->dn + (size_t)expert * L->dn_bytes, ctx->s.staging, L->H, L->Ipad, ctx->stream));
-  HIP_TRY(hipMemcpyAsync(down, ctx->s.staging, L->dn_bytes, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
-  return RMOE_OK;
+  const Stretch parts[2] = {{L->gu + (size_t)expert * L->gu_bytes, 2 * L->I, L->H, RMOE_FMT_Q4NX,
+                             static_cast<uint8_t*>(gate_up), L->gu_bytes},
+                            {L->dn + (size_t)expert * L->dn_bytes, L->H, L->Ipad, L->dn_fmt,
+                             static_cast<uint8_t*>(down), L->dn_bytes}};
+  return has_gu ? download_chunked(ctx, parts, 2) : download_chunked(ctx, parts + 1, 1);
 }
 
 static int set_router_common(rmoe_ctx* ctx, RmoeLayer* L, const void* w, bool w_on_device, const float* bias, int score,
@@ -884,18 +954,24 @@ int rmoe_moe_experts(rmoe_ctx* ctx, int layer, const uint16_t* x, const int32_t*
   TRY(check_decode_shape(*L, k, layer));
   HIP_TRY(hipSetDevice(ctx->device));
   TRY(reserve_layer(ctx, *L, 1, k));
-  const size_t xb = align_up((size_t)L->H * 2, 256);
+  // x, ids and weights go to the device by one launch that reads the pinned input slot, and
+  // the down kernel writes its output to the pinned output slot.
+  const size_t xb = align_up((size_t)L->H * 2, 256), in = xb + 128;
+  if (in > kPinnedIo) return fail(RMOE_EINVAL, "hidden size %d is too large", L->H);
   uint8_t* io;
-  TRY(io_area(ctx, 2 * xb + 256, &io));
-  uint16_t* xd = (uint16_t*)io;
-  uint16_t* od = (uint16_t*)(io + xb);
-  HIP_TRY(hipMemcpyAsync(xd, x, (size_t)L->H * 2, hipMemcpyHostToDevice, ctx->stream));
-  HIP_TRY(hipMemcpyAsync(ctx->s.ids, top_ids, (size_t)k * 4, hipMemcpyHostToDevice, ctx->stream));
-  HIP_TRY(hipMemcpyAsync(ctx->s.wts, top_weights, (size_t)k * 4, hipMemcpyHostToDevice, ctx->stream));
-  HIP_TRY(rmoe::launch_moe_decode(*L, xd, ctx->s.ids, ctx->s.wts, k, false, act, gate_beta, value_beta, false, nullptr,
-                                  od, ctx->s, ctx->stream));
-  HIP_TRY(hipMemcpyAsync(out, od, (size_t)L->H * 2, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
+  TRY(io_area(ctx, in, &io));
+  memcpy(ctx->pinned, x, (size_t)L->H * 2);
+  memcpy(ctx->pinned + xb, top_ids, (size_t)k * 4);
+  memcpy(ctx->pinned + xb + 64, top_weights, (size_t)k * 4);
+  uint16_t* od = reinterpret_cast<uint16_t*>(ctx->pinned_dev + kPinnedIo);
+  hipError_t e = rmoe::launch_copy16(ctx->pinned_dev, io, in, ctx->stream);
+  if (e == hipSuccess)
+    e = rmoe::launch_moe_decode(*L, (uint16_t*)io, (int32_t*)(io + xb), (float*)(io + xb + 64), k, false, act,
+                                gate_beta, value_beta, false, nullptr, od, ctx->s, ctx->stream);
+  const hipError_t es = hipStreamSynchronize(ctx->stream);  // also on failure: the slots are in use until then
+  HIP_TRY(e);
+  HIP_TRY(es);
+  memcpy(out, ctx->pinned + kPinnedIo, (size_t)L->H * 2);
   return RMOE_OK;
 }
 

@@ -409,6 +409,11 @@ struct rmoe_ctx {
   int next_handle = 1;
   std::map<int, RmoeLayer> layers;
   RmoeScratch s;
+  // Pinned host memory the device reads and writes (host entry points): two slots for the
+  // inputs and the output of one token, four for the chunks of a download.
+  uint8_t* pinned = nullptr;      // host address
+  uint8_t* pinned_dev = nullptr;  // the same memory's device address
+  hipEvent_t chunk_done[4] = {};
   unsigned stack_wait_limit = 0;  // polls before a wait of the decode stack gives up (0: default)
 };
 
@@ -417,7 +422,11 @@ struct rmoe_ctx {
 namespace rmoe {
 
 hipError_t launch_relayout_in(const uint8_t* packed, uint8_t* tiles, int M, int K, hipStream_t st);
-hipError_t launch_relayout_out(const uint8_t* tiles, uint8_t* packed, int M, int K, hipStream_t st);
+// Blocks [first, first + n) of the output, kRelayoutBytes each in order, to packed
+// (n = 0: all from first on).
+constexpr size_t kRelayoutBytes = 2 * kTileBytes;
+hipError_t launch_relayout_out(const uint8_t* tiles, uint8_t* packed, int M, int K, size_t first, size_t n,
+                               hipStream_t st);
 // Rows [row0, row0 + M) of a tile matrix Kt wide from a row-major Q4_K tensor [M, K].
 hipError_t launch_q4k_to_tiles(const uint8_t* q4k, int M, int K, uint8_t* tiles, int Kt, int row0, hipStream_t st);
 hipError_t launch_quantize(const float* w, int M, int K, int ld, int k_valid, uint8_t* tiles, int* err,
@@ -450,6 +459,8 @@ hipError_t launch_route(const RmoeLayer& L, const uint16_t* x, int T, int32_t* i
 // with its own copy of the one-token scratch.
 // out_routed (may be null) gets RTNE of the routed sum; out gets the full combine
 // (routed + shared, + x when residual).
+// n bytes (a multiple of 16) from src to dst, both 16-byte aligned and reachable by the device.
+hipError_t launch_copy16(const void* src, void* dst, size_t n, hipStream_t st);
 hipError_t launch_moe_decode(const RmoeLayer& L, const uint16_t* x, const int32_t* ids, const float* wts, int k,
                              bool with_shared, int act, float gb, float vb, bool residual, uint16_t* out,
                              uint16_t* out_routed, RmoeScratch& s, hipStream_t st, int stages = 3, int ntok = 1);

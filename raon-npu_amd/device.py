@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from ._lib import ACT_SITU, ACT_SWIGLU, BUNDLE_B1, BUNDLE_B2, PART_DOWN, PART_GATE_UP, SCORE_SIGMOID, SCORE_SOFTMAX, call, ptr
+from ._lib import ACT_SITU, ACT_SWIGLU, BUNDLE_B1, BUNDLE_B2, PART_DOWN, PART_GATE_UP, SCORE_SIGMOID, SCORE_SOFTMAX, call, new_bytes, ptr
 from .geometry import MoeGeometry
 
 
@@ -209,9 +209,9 @@ class Matrix:
         return self.M * self.K * self._BITS[self.fmt] // 8
 
     def download(self) -> bytes:
-        out = np.empty(self.nbytes, dtype=np.uint8)
-        call("rmoe_matrix_download", self.ctx.handle, self.handle, ptr(out), out.size)
-        return out.tobytes()
+        out, addr = new_bytes(self.nbytes)
+        call("rmoe_matrix_download", self.ctx.handle, self.handle, addr, len(out))
+        return out
 
     def linear(self, x: np.ndarray) -> np.ndarray:
         """bf16 ``x[..., K_in]`` (K_in <= K, zero padded) -> bf16 ``[..., M]``."""
@@ -315,11 +315,10 @@ class MoeLayer:
         """(gate_up, down) GEMV bytes of one expert; gate_up is b"" for the shared expert
         of a weights-d layer, whose gate/up lives outside the layer."""
         no_gu = self.d_layout and int(expert) == self.geom.n_routed
-        gu = None if no_gu else np.empty(self.gu_expert_bytes, np.uint8)
-        dn = np.empty(self.dn_expert_bytes, np.uint8)
-        call("rmoe_layer_download_expert", self.ctx.handle, self.layer, int(expert), ptr(gu), 0 if no_gu else gu.size,
-             ptr(dn), dn.size)
-        return (b"" if no_gu else gu.tobytes()), dn.tobytes()
+        gu, gu_ptr = (b"", None) if no_gu else new_bytes(self.gu_expert_bytes)
+        dn, dn_ptr = new_bytes(self.dn_expert_bytes)
+        call("rmoe_layer_download_expert", self.ctx.handle, self.layer, int(expert), gu_ptr, len(gu), dn_ptr, len(dn))
+        return gu, dn
 
     def set_router(self, weight_bf16, bias=None, score: str = "softmax", renormalize: bool = True, scaling: float = 1.0):
         code = {"sigmoid": SCORE_SIGMOID, "softmax": SCORE_SOFTMAX}[score]

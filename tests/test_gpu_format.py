@@ -92,3 +92,16 @@ def test_quantize_and_download_tiles(gpu_ctx, M, K, offset):
     mat = gpu_ctx.upload_matrix(blob, M, K)
     assert bytes(mat.download()) == blob
     mat.free()
+
+
+# q4nx: 51 blocks of 10,240 bytes are one chunk of the download; 50, 52, 204 (the whole ring)
+# and 206 blocks.  bfp16: the same sizes at nine bits, chunks cut anywhere.
+@pytest.mark.parametrize("fmt, bits", [("q4nx", 5), ("bfp16", 9)])
+@pytest.mark.parametrize("blocks", [50, 52, 204, 206])
+def test_download_chunk_edges(gpu_ctx, fmt, bits, blocks):
+    M, K = 128, 128 * blocks
+    blob = np.random.default_rng(blocks).integers(0, 256, M * K * bits // 8, dtype=np.uint8).tobytes()
+    mat = gpu_ctx.upload_matrix(blob, M, K, fmt=fmt)
+    for _ in range(2):
+        assert mat.download() == blob
+    mat.free()

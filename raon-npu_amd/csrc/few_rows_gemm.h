@@ -9,17 +9,25 @@
 // registers (one 16-byte load per lane and fragment of 16 rows), stages the tile's
 // activation rows in an LDS region of its own (WaveRows), and several workgroups are
 // resident per CU, each hiding the others' prologue and load rounds.
+// Of a weight tile's 5 KB, 1 KB are scales and mins, which the correction needs before the K
+// loop: their scales stay in LDS from there on (2 KB per K tile, 32 to 40 KB per workgroup;
+// reading them again beside the codes cost 3 to 7 % of gate/up), and the first block of them
+// is requested with the first codes, before the row indices are known.
 // Kernel times against grouped_gemm_kernel, gate/up and down: H=2048, I=768, 445 tokens 95 ->
-// 84 and 57 -> 48 us; H=2560, I=1088, 32 tokens 108 -> 82 and 61 -> 45 us, 256 tokens 142 ->
-// 116 and (bfp16) 139 -> 99 us: 4.2 to 4.7 TB/s of expert weights over the whole kernel, ~7
-// TB/s inside the K loops; a workgroup spends ~10 of its ~35 us on the rows, the correction
-// and the first loads.  Tiles of 32 rows instead of 48 cost 3 to 8 % at 445 tokens, three
-// workgroups per CU (168 registers, spills) 10 to 30 %, the first weight tiles requested
-// after the correction instead of first 5 to 45 %.
+// 80 and 57 -> 47 us; H=2560, I=1088, 32 tokens 108 -> 79 and 61 -> 44 us, 256 tokens 142 ->
+// 119 and (bfp16) 139 -> 104 us: 4.2 to 4.9 TB/s of expert weights over the whole kernel.  The
+// rest is the workgroups' last round: 828 of them in 512 places at 445 tokens.  Tiles of 32
+// rows instead of 48 cost 3 to 8 % at 445 tokens, three workgroups per CU (168 registers,
+// spills) 10 to 30 %, the first weight tiles requested after the correction instead of first
+// 5 to 45 %.
 #pragma once
 
 // A barrier that waits for the wave's LDS accesses only.
 __device__ __forceinline__ void few_rows_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+constexpr int kFewStageBytes = 2 * kBMFew * 256;                  // two K tiles of activation rows
+constexpr int kFewGateUpOut = 3 * kBMFew * kOutStride * 2;         // gate, up and h of SiTU
+constexpr int kFewDownOut = kBMFew * 264 * 2;
 
 // One tile of 16 MF rows by 256 weight rows.  Gate/up: units 128 nt + 32 w .. +31 in wave w
 // (fragments 0, 1 gate, 2, 3 up); down: output columns 256 nt + 64 w .. +63.
@@ -48,12 +56,12 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     if (dead) wrow[f] = 0;
     wf[f] = W + (size_t)(wrow[f] / kTileRows) * wkt * kTB + (wrow[f] % kTileRows) * 16;
   }
-  // Weights of one K tile.  q4nx: codes of (row l16, group lq) and the scale | min word;
+  // Weights of one K tile.  q4nx: codes of (row l16, group lq), the scales come from LDS;
   // bfp16: mantissas of columns 32 lq .. +31 and their four exponents.  The first two tiles
   // depend on the tile entry only: requested before anything else.
   struct WTile {
     uint4 c[NF][kB16 ? 2 : 1];
-    uint32_t s[NF];
+    uint32_t s[kB16 ? NF : 1];
   };
   auto load_w = [&](int kt, WTile& w) {
     const bool live = kt < nkt && !dead;
@@ -66,22 +74,97 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
         w.s[f] = wg_load<uint32_t>(p + kB16MantBytes, live ? 16u * l16 + 4u * lq : 0u);
       } else {
         w.c[f][0] = wg_load_weights<true>(p, live ? 1024u * lq + 16u * l16 : 0u);
-        w.s[f] = wg_load<uint32_t>(p + kCodeBytes, live ? 16u * l16 + 4u * lq : 0u);
       }
     }
     asm volatile("" ::: "memory");  // keeps the loads where they are
   };
   WTile wa, wb, wc;
+  // Correction operands of a block of 32 groups: the scale | min words of groups 32 blk +
+  // 8 lq .. +7 of weight row l16, and the group sums of activation row l16 for them.
+  const int G = a.K / 32, Gp = sum_planes_gp(G), nblk = kB16 ? 0 : (G + 31) / 32;
+  struct Coef {
+    uint4 c[NF][2];
+  };
+  struct Sums {
+    uint4 s[MF][3];
+  };
+  auto load_c = [&](int blk, Coef& b) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int kt = 8 * blk + 2 * lq + h;
+        b.c[f][h] = wg_load<uint4>(wf[f] + kCodeBytes, (uint32_t)((4 * kt < G ? kt : 0) * kTB + 16 * l16));
+      }
+    asm volatile("" ::: "memory");
+  };
+  [[maybe_unused]] Coef ca, cb;
 
   // Source row of each tile row (rows past the tile repeat its first row and are not
-  // stored) and its power-of-two exponent; a down row's is the largest of its chunks'.
-  int my_src = 0, my_e = 0, my_d = 0;
+  // stored).  A down tile's rows lie one after another; a gate/up tile's token rows are
+  // loaded, with the first weights in flight behind them.  (The barriers here wait for LDS
+  // only: __syncthreads() would also wait for the weights.)
+  const int my_row = row0 + (tid < nrows ? tid : 0);
+  int my_src = my_row;
+  if constexpr (!kDown) {
+    if (tid < 16 * MF) my_src = e < a.n_routed ? a.order[my_row] : my_row - a.shared_base;
+  }
+  if constexpr (!kB16) load_c(0, ca);
+  load_w(0, wa);
+  load_w(1, wb);
+  if constexpr (!kDown) {
+    if (tid < 16 * MF) rowidx[tid] = my_src = e < a.n_routed ? my_src / a.k_routes : my_src;
+    few_rows_barrier();
+  }
+  auto src_row = [&](int r) { return kDown ? row0 + (r < nrows ? r : 0) : rowidx[r]; };
+
+  // Activation rows: thread t brings 16-byte chunk t % 16 of rows t / 16 + 16 i of a K tile,
+  // through registers into LDS chunk (t % 16) ^ (row % 16) of the row (as WaveRows).
+  const int xrow = tid >> 4;
+  uint32_t xoff[MF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+    xoff[i] = (uint32_t)src_row(xrow + 16 * i) * (uint32_t)(2 * a.K) + 16u * (uint32_t)(tid & 15);
+  const uint32_t xwr = 256u * xrow + 16u * (uint32_t)((tid & 15) ^ xrow);
+  uint4 xr[MF];
+  auto load_x = [&](int kt) {
+    const uint8_t* xb = reinterpret_cast<const uint8_t*>(a.src) + (size_t)min(kt, nkt - 1) * 256;
+#pragma unroll
+    for (int i = 0; i < MF; ++i) xr[i] = wg_load<uint4>(xb, kt < nkt ? xoff[i] : 0u);
+  };
+  Sums sa;
+  [[maybe_unused]] Sums sb;
+  uint32_t srow[MF];
+#pragma unroll
+  for (int m = 0; m < MF; ++m) srow[m] = kB16 ? 0u : (uint32_t)src_row(16 * m + l16) * (uint32_t)(6 * Gp);
+  auto load_s = [&](int blk, Sums& b) {
+    const int gl = 32 * blk + 8 * lq;
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        b.s[m][p] = wg_load<uint4>(reinterpret_cast<const uint8_t*>(a.ssum + p * Gp),
+                                   srow[m] + 2u * (uint32_t)(gl < Gp ? gl : 0));
+    asm volatile("" ::: "memory");
+  };
+  if constexpr (!kB16) load_s(0, sa);
+  // What is in flight during the correction, as far as registers go (a spill is never worth
+  // it here: one has corrupted row addresses).  256 registers with these, none spilled.
+  constexpr bool kCoefAhead = MF <= 2, kSumsAhead = MF <= 1, kRowsAhead = MF <= 1;
+  if constexpr (kRowsAhead) {
+    load_x(0);
+    asm volatile("" ::: "memory");
+  }
+  if constexpr (!kB16 && kCoefAhead) {
+    if (nblk > 1) load_c(1, cb);
+  }
+  // Power-of-two exponent of each row; a down row's is the largest of its chunks'.
+  int my_e = 0, my_d = 0;
   if (tid < 16 * MF) {
-    const int p = row0 + (tid < nrows ? tid : 0);
     if constexpr (kDown) {
       int emax = -128, emin = 127;
       for (int c0 = 0; c0 < a.K / 128; c0 += 16) {
-        const uint4 v = *reinterpret_cast<const uint4*>(a.hexp + (size_t)p * eso + c0);
+        const uint4 v = *reinterpret_cast<const uint4*>(a.hexp + (size_t)my_row * eso + c0);
         const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int c = 0; c < 16; ++c)
@@ -91,48 +174,25 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
             emin = min(emin, ec);
           }
       }
-      my_src = p;
       my_e = emax;
       my_d = emin != emax ? 1 : 0;
     } else {
-      my_src = e < a.n_routed ? a.order[p] / a.k_routes : p - a.shared_base;
       my_e = a.aexp[my_src];
     }
-  }
-  load_w(0, wa);
-  load_w(1, wb);
-  if (tid < 16 * MF) {
-    rowidx[tid] = my_src;
     row_e[tid] = (int8_t)my_e;
   }
-  // (Rows are wave 0's: its vote is the tile's.  The barriers here wait for LDS only:
-  // __syncthreads() would also wait for the weights.)
-  const unsigned long long vote = __ballot(my_d != 0);
+  const unsigned long long vote = __ballot(my_d != 0);  // rows are wave 0's: its vote is the tile's
   if (tid == 0) *differ = vote ? 1 : 0;
   few_rows_barrier();
   const bool rescale = kDown && *differ != 0;
 
-  // Activation rows: thread t brings 16-byte chunk t % 16 of rows t / 16 + 16 i of a K tile,
-  // through registers into LDS chunk (t % 16) ^ (row % 16) of the row (as WaveRows).
-  const int xrow = tid >> 4;
-  uint32_t xoff[MF];
-#pragma unroll
-  for (int i = 0; i < MF; ++i)
-    xoff[i] = (uint32_t)rowidx[xrow + 16 * i] * (uint32_t)(2 * a.K) + 16u * (uint32_t)(tid & 15);
-  const uint32_t xwr = 256u * xrow + 16u * (uint32_t)((tid & 15) ^ xrow);
-  uint4 xr[MF];
-  auto load_x = [&](int kt) {
-    const uint8_t* xb = reinterpret_cast<const uint8_t*>(a.src) + (size_t)min(kt, nkt - 1) * 256;
-#pragma unroll
-    for (int i = 0; i < MF; ++i) xr[i] = wg_load<uint4>(xb, kt < nkt ? xoff[i] : 0u);
-  };
   auto h2 = [](uint32_t v) { return __builtin_bit_cast(f16x2_t, v); };
   auto u2 = [](f16x2_t v) { return __builtin_bit_cast(uint32_t, v); };
   auto store_x = [&](int kt) {
     if (rescale && kt < nkt) {  // a chunk below its row's exponent (rare), as h_unify_kernel
 #pragma unroll
       for (int i = 0; i < MF; ++i) {
-        const int r = xrow + 16 * i, d = (int)a.hexp[(size_t)rowidx[r] * eso + kt] - (int)row_e[r];
+        const int r = xrow + 16 * i, d = (int)a.hexp[(size_t)src_row(r) * eso + kt] - (int)row_e[r];
         if (d == 0) continue;
         uint32_t v[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
 #pragma unroll
@@ -155,11 +215,12 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[m][f] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // The wave's scales, for the K loop: [K tile][fragment][row][group] bf16 in LDS.
+  uint8_t* wsc = lds + kFewStageBytes + (size_t)wave * wkt * (NF * 128) + 8 * l16;
   int fx[NF];
   [[maybe_unused]] int emax_w[NF];
   {
     if constexpr (kB16) {
-      load_x(0);
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         emax_w[f] = a.rowexp[(size_t)e * a.N_total + wrow[f] + l16];
@@ -167,38 +228,20 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
       }
     } else {
       // Correction: acc += sum_g (min + 8 scale)[r, g] S[m, g], six products per block of 32
-      // groups on bf16 MFMA in gemm_tile's order.  Lane (l16, lq) takes groups 32 blk + 8 lq
-      // .. +7 of weight row l16 and of activation row l16.
-      const int G = a.K / 32, Gp = sum_planes_gp(G), nblk = (G + 31) / 32;
-      struct CBlk {
-        uint4 c[NF][2], s[MF][3];
-      };
-      uint32_t srow[MF];
-#pragma unroll
-      for (int m = 0; m < MF; ++m) srow[m] = (uint32_t)rowidx[16 * m + l16] * (uint32_t)(6 * Gp);
-      auto load_blk = [&](int blk, CBlk& b) {
-        const int gl = 32 * blk + 8 * lq;
-#pragma unroll
-        for (int f = 0; f < NF; ++f)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int kt = gl / 4 + h;
-            b.c[f][h] = wg_load<uint4>(wf[f] + kCodeBytes, (uint32_t)((4 * kt < G ? kt : 0) * kTB + 16 * l16));
-          }
-#pragma unroll
-        for (int m = 0; m < MF; ++m)
-#pragma unroll
-          for (int p = 0; p < 3; ++p)
-            b.s[m][p] = wg_load<uint4>(reinterpret_cast<const uint8_t*>(a.ssum + p * Gp),
-                                       srow[m] + 2u * (uint32_t)(gl < Gp ? gl : 0));
-      };
+      // groups on bf16 MFMA in gemm_tile's order.
       uint32_t smax[NF] = {0u, 0u, 0u, 0u};
-      auto corr_blk = [&](int blk, const CBlk& b) {
+      auto corr_blk = [&](int blk, const Coef& b, const Sums& s) {
         const int gl = 32 * blk + 8 * lq;
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
           const uint32_t sv[8] = {b.c[f][0].x, b.c[f][0].y, b.c[f][0].z, b.c[f][0].w,
                                   b.c[f][1].x, b.c[f][1].y, b.c[f][1].z, b.c[f][1].w};
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            if (gl + 4 * h < G)
+              *reinterpret_cast<uint2*>(wsc + ((8 * blk + 2 * lq + h) * NF + f) * 128) =
+                  make_uint2(__builtin_amdgcn_perm(sv[4 * h + 1], sv[4 * h], 0x05040100u),
+                             __builtin_amdgcn_perm(sv[4 * h + 3], sv[4 * h + 2], 0x05040100u));
           uint32_t w[8];
           float s8[8];
 #pragma unroll
@@ -217,30 +260,31 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
           for (int p = 0; p < 6; ++p)
 #pragma unroll
             for (int m = 0; m < MF; ++m)
-              acc[m][f] = mfma16(b.s[m][2 - p / 2], (p & 1) ? bsc8 : bmin, acc[m][f]);
+              acc[m][f] = mfma16(s.s[m][2 - p / 2], (p & 1) ? bsc8 : bmin, acc[m][f]);
         }
       };
-      if constexpr (MF <= 1) {
-        CBlk ca, cb;
-        load_blk(0, ca);
+      if constexpr (kCoefAhead) {
 #pragma unroll 1
         for (int blk = 0; blk < nblk; blk += 2) {
-          if (blk + 1 < nblk) load_blk(blk + 1, cb);
-          else load_x(0);
-          corr_blk(blk, ca);
+          if (kSumsAhead && blk + 1 < nblk) load_s(blk + 1, sb);
+          corr_blk(blk, ca, sa);
           if (blk + 1 < nblk) {
-            if (blk + 2 < nblk) load_blk(blk + 2, ca);
-            else load_x(0);
-            corr_blk(blk + 1, cb);
+            if (!kSumsAhead) load_s(blk + 1, sa);
+            if (blk + 2 < nblk) load_c(blk + 2, ca);
+            if (kSumsAhead && blk + 2 < nblk) load_s(blk + 2, sa);
+            corr_blk(blk + 1, cb, kSumsAhead ? sb : sa);
+            if (!kSumsAhead && blk + 2 < nblk) load_s(blk + 2, sa);
+            if (blk + 3 < nblk) load_c(blk + 3, cb);
           }
         }
-      } else {  // registers for one block: two would spill, which has corrupted row addresses here
+      } else {
 #pragma unroll 1
         for (int blk = 0; blk < nblk; ++blk) {
-          CBlk c;
-          load_blk(blk, c);
-          if (blk + 1 == nblk) load_x(0);
-          corr_blk(blk, c);
+          corr_blk(blk, ca, sa);
+          if (blk + 1 < nblk) {
+            load_c(blk + 1, ca);
+            load_s(blk + 1, sa);
+          }
         }
       }
       // Weight-row exponents, as in gemm_tile: the largest scale lands in [2^11, 2^12).
@@ -265,6 +309,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
         }
       }
     };
+    if constexpr (!kRowsAhead) load_x(0);
     if constexpr (!kB16) scale_rows(-1);
 
     // K loop: MFMA j takes columns 32 lq + 8j .. +7 from lane quarter lq, the activations'
@@ -287,7 +332,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
       if constexpr (!kB16) {
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
-          const float sc = bf16_to_f32(w.s[f] & 0xffffu);
+          const float sc = bf16_to_f32(*reinterpret_cast<const uint16_t*>(wsc + (kt * NF + f) * 128 + 2 * lq));
           const float v1 = __builtin_amdgcn_ldexpf(sc, -fx[f]), v16 = __builtin_amdgcn_ldexpf(sc, -fx[f] - 4);
           s1[f] = __builtin_bit_cast(f16x2_t, __builtin_amdgcn_cvt_pkrtz(v1, v1));
           s16[f] = __builtin_bit_cast(f16x2_t, __builtin_amdgcn_cvt_pkrtz(v16, v16));
@@ -435,12 +480,18 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     for (int r = tid >> 4; r < nrows; r += 16) zero_row_padding(a, row0 + r, tid & 15, 16);
 }
 
+// Dynamic LDS: the stages and, with q4nx weights, the four waves' scales (2 KB per K tile);
+// then, in the same place, the epilogue staging.
+static size_t few_rows_lds(const GemmArgs& a, bool b16) {
+  const size_t loop = kFewStageBytes + (b16 ? 0 : (size_t)4 * (a.K / kTileCols) * 512);
+  return std::max(loop, (size_t)(a.mode == 0 ? kFewGateUpOut : kFewDownOut));
+}
+
 // Grid: as grouped_gemm_kernel's, 256 threads.  XCD x takes a contiguous eighth of each
 // class's tiles, the largest first.
 template <bool kDown, bool kB16>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void few_rows_gemm_kernel(GemmArgs a, int cap) {
-  // Two stages of 48 rows, then the epilogue staging (the largest: three 48-row SiTU tiles).
-  __shared__ __attribute__((aligned(16))) uint8_t lds[3 * kBMFew * kOutStride * 2];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // few_rows_lds() bytes
   __shared__ int rowidx[kBMFew];
   __shared__ __attribute__((aligned(16))) int8_t row_e[kBMFew];
   __shared__ int differ;

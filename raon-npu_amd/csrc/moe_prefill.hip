@@ -1592,18 +1592,29 @@ static hipError_t launch_grouped(GemmArgs a, uint32_t* tiles, int* ntiles, int c
   const int per2 = 8 * ((a.n_tiles * cap + 7) / 8), per01 = 8 * ((a.n_tiles * small + 7) / 8);
   if (few) {
     const dim3 grid(per2 + 2 * per01), block(256);
-    if (a.mode == 0)
-      hipLaunchKernelGGL((few_rows_gemm_kernel<false, false>), grid, block, 0, st, a, cap);
-    else if (b16)
-      hipLaunchKernelGGL((few_rows_gemm_kernel<true, true>), grid, block, 0, st, a, cap);
-    else
-      hipLaunchKernelGGL((few_rows_gemm_kernel<true, false>), grid, block, 0, st, a, cap);
+    const size_t lds = few_rows_lds(a, b16);
+    auto* kernel = a.mode == 0 ? few_rows_gemm_kernel<false, false>
+                   : b16       ? few_rows_gemm_kernel<true, true>
+                               : few_rows_gemm_kernel<true, false>;
+    hipLaunchKernelGGL(kernel, grid, block, lds, st, a, cap);
   } else if (b16) {
     hipLaunchKernelGGL((grouped_gemm_kernel<7, true>), dim3(per2 + 2 * per01), dim3(512), 0, st, a, cap);
   } else {
     hipLaunchKernelGGL((grouped_gemm_kernel<7, false>), dim3(per2 + 2 * per01), dim3(512), 0, st, a, cap);
   }
   return hipGetLastError();
+}
+
+// Allow the few-rows kernels the dynamic LDS of the widest layer (K = 8192).
+hipError_t prefill_setup() {
+  const int lds = kFewStageBytes + 4 * (8192 / kTileCols) * 512;
+  const void* fns[3] = {(const void*)few_rows_gemm_kernel<false, false>, (const void*)few_rows_gemm_kernel<true, true>,
+                        (const void*)few_rows_gemm_kernel<true, false>};
+  for (const void* f : fns) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // Whether the batch's groups are short enough for few_rows_gemm_kernel: on average at most

@@ -381,10 +381,11 @@ int rmoe_create(int device, rmoe_ctx** out) {
   }
   bool ok = hipHostMalloc((void**)&ctx->pinned, kPinnedBytes, hipHostMallocDefault) == hipSuccess &&
             hipHostGetDevicePointer((void**)&ctx->pinned_dev, ctx->pinned, 0) == hipSuccess;
+  ok = ok && rmoe::prefill_setup() == hipSuccess;
   for (hipEvent_t& ev : ctx->chunk_done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
   if (!ok) {
     free_base(ctx);
-    return fail(RMOE_ENOMEM, "%zu bytes of pinned host memory failed", kPinnedBytes);
+    return fail(RMOE_EDEVICE, "setting up device %d with %zu bytes of pinned host memory failed", device, kPinnedBytes);
   }
   // The persistent decode kernel runs one workgroup per CU and needs all of them
   // resident at once.

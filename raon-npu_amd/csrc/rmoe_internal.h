@@ -483,6 +483,7 @@ hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int3
 // and writes ids_out/wts_out; otherwise ids_in/wts_in are used.  With shared_gu the
 // shared expert's gate/up is taken from it, otherwise computed from x.  Any of out /
 // routed / shared_down may be null.  scratch: prefill_scratch_bytes(L, T) bytes.
+hipError_t prefill_setup();  // once per device before the first prefill
 size_t prefill_scratch_bytes(const RmoeLayer& L, int T);
 hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, const int32_t* ids_in, const float* wts_in,
                               int32_t* ids_out, float* wts_out, const uint16_t* shared_gu, int act, float gb, float vb,

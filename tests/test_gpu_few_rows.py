@@ -86,3 +86,23 @@ def test_few_rows_prefill_equals_many_rows(gpu_ctx):
     for T in (1, 16, 47, FEW):
         np.testing.assert_array_equal(run(T), want[:T], err_msg=f"T={T}")
     lyr.free()
+
+
+# Blocks of 32 groups in the correction: one, two and a quarter, three and a quarter, eight (the
+# widest layer, whose scales fill LDS); rows per group for each tile class.
+@pytest.mark.parametrize("hidden", [1024, 2304, 3328, 8192])
+def test_few_rows_widths(gpu_ctx, hidden):
+    geom = G.MoeGeometry(hidden=hidden, inter=64, n_routed=4, n_shared=1, top_k=1)
+    syn = make_layer(geom, seed=77)
+    lyr = gpu_ctx.create_layer(1702, geom)
+    lyr.upload_experts(syn.gate_up, syn.down)
+    x = random_tokens(260, hidden, 78)
+    ids = np.repeat(np.arange(4), [5, 16, 30, 209]).astype(np.int32)[:, None]
+    wts = np.ones(ids.shape, np.float32)
+    sgu = random_tokens(260, 128, 79)
+    want_r, want_s = lyr.moe_experts_grouped(x, ids, wts, sgu)  # 65 rows per expert: the general kernel
+    for T in (5, 51, 98):  # the last groups hold 5, 30 and 47 rows
+        r, s = lyr.moe_experts_grouped(x[:T], ids[:T], wts[:T], sgu[:T])
+        np.testing.assert_array_equal(r, want_r[:T], err_msg=f"routed, T={T}")
+        np.testing.assert_array_equal(s, want_s[:T], err_msg=f"shared, T={T}")
+    lyr.free()

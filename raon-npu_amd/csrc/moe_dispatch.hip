@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void dispatch_count_kernel(const int32_t* __re
 }
 
 // counts[c][e]: assignments of chunk c routed to expert e.  Workgroup c also writes
-// offsets[e] (E + 1 entries) when c == 0.
+// offsets[e] (E + 1 entries) when c == 0; workgroup nchunks (launched with tiles) the tile table.
 __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __restrict__ ids, int n, int E,
                                                                const int32_t* __restrict__ counts, int nchunks,
                                                                int32_t* __restrict__ offsets,
@@ -66,6 +66,22 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __
   if (lane == 63) wsum[wave] = incl;
   unsigned long long same[4];
   __syncthreads();
+  // The grouped GEMM's tile table (when asked for): routed group e holds sorted rows
+  // [offset, offset + total); the shared group (shared_rows > 0) starts at row n (after
+  // every assignment, whether or not its id was valid), where the GEMM places it.  A
+  // workgroup of its own past the chunks writes it, beside the scatter instead of after the
+  // first chunk's (11.6 -> 10.1 us at 6,700 x 8 assignments, 7.2 -> 5.3 at 445 x 8).
+  if (c == nchunks) {
+    __shared__ int tsum[kTileClasses][4];
+    int gb = n;
+    if (tid < E) {
+      gb = incl - total;
+      for (int w = 0; w < wave; ++w) gb += wsum[w];
+    }
+    tile_table_block<4>(tid, E + (shared_rows > 0 ? 1 : 0), gb, gb + (tid < E ? total : shared_rows), tiles, ntiles,
+                        cap, bm, tsum);
+    return;
+  }
   // Lanes of one round with the same expert agree on every bit of the id.
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -112,15 +128,6 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int32_t* __
     }
     if (same[j] && (same[j] >> lane) == 1ull) slot[wave][e] += __popcll(same[j]);
   }
-  // The grouped GEMM's tile table (when asked for): routed group e holds sorted rows
-  // [offset, offset + total); the shared group (shared_rows > 0) starts at row n (after
-  // every assignment, whether or not its id was valid), where the GEMM places it.
-  if (c == 0 && tiles) {
-    __shared__ int tsum[kTileClasses][4];
-    const int ng = E + (shared_rows > 0 ? 1 : 0);
-    const int gb = tid < E ? offset : n;
-    tile_table_block<4>(tid, ng, gb, gb + (tid < E ? total : shared_rows), tiles, ntiles, cap, bm, tsum);
-  }
 }
 
 }  // namespace
@@ -139,8 +146,8 @@ hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int3
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(dispatch_scatter_kernel, dim3(nchunks), dim3(256), 0, st, ids, n, n_experts, s.chunk_counts,
-                     nchunks, offsets, order, inv, tiles, ntiles, cap, shared_rows, bm);
+  hipLaunchKernelGGL(dispatch_scatter_kernel, dim3(nchunks + (tiles ? 1 : 0)), dim3(256), 0, st, ids, n, n_experts,
+                     s.chunk_counts, nchunks, offsets, order, inv, tiles, ntiles, cap, shared_rows, bm);
   return hipGetLastError();
 }
 

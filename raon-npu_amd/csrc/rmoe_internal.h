@@ -279,8 +279,8 @@ __device__ __forceinline__ void tile_table_block(int e, int ng, int b, int end, 
   int full = 0, cnt[kTileClasses] = {0, 0, 0};
   if (e < ng) {
     const int c0 = bm == kBM ? 32 : 16, c1 = bm == kBM ? 64 : 32;  // most rows of classes 0 and 1
-    full = (end - b) / bm;
-    const int rem = (end - b) % bm;
+    full = bm == kBM ? (end - b) / kBM : (end - b) / kBMFew;
+    const int rem = (end - b) - full * bm;
     cnt[2] = full + (rem > c1 ? 1 : 0);
     cnt[1] = (rem > c0 && rem <= c1) ? 1 : 0;
     cnt[0] = (rem > 0 && rem <= c0) ? 1 : 0;

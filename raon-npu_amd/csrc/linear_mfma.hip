@@ -93,6 +93,12 @@ __global__ __launch_bounds__(512) void linear_mfma_kernel(LinMfmaArgs a) {
   }
 }
 
+// Dynamic LDS of W waves: their activation regions, then in the same place their partial sums.
+constexpr size_t linear_lds(int MF, int NF, int W) {
+  const size_t sums = (size_t)16 * MF * (16 * NF + kPad) * 4, rows = (size_t)4096 * MF;
+  return W * (sums > rows ? sums : rows);
+}
+
 template <int kFmt, int MF, int NF, int XI>
 hipError_t launch(LinMfmaArgs a, hipStream_t st) {
   // Waves per workgroup: four, eight for 64 K tiles and more ([2560, 12032], one token:
@@ -101,7 +107,7 @@ hipError_t launch(LinMfmaArgs a, hipStream_t st) {
   const int nkt = a.K / kTileCols, W = std::min(nkt, nkt >= 64 ? 8 : 4);
   a.n_mt = (a.T + 16 * MF - 1) / (16 * MF);
   a.n_nt = a.M / (16 * NF);
-  const size_t lds = (size_t)W * std::max(16 * MF * (16 * NF + kPad) * 4, 4096 * MF);
+  const size_t lds = linear_lds(MF, NF, W);
   const size_t total = (size_t)a.n_mt * a.n_nt;
   hipLaunchKernelGGL((linear_mfma_kernel<kFmt, MF, NF, XI>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(64 * W), lds,
                      st, a);
@@ -143,6 +149,17 @@ bool linear_mfma_ok(int M, int K, const uint16_t* x, int T, const uint16_t* y) {
   // that fits its counter.
   return (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0 &&
          (size_t)T * K * 2 < ((size_t)1 << 32) && ((size_t)T + 15) / 16 * (M / 16) < ((size_t)1 << 28);
+}
+
+// Allow the 32 x 64 tiles of eight waves their 68 KB of dynamic LDS (the others stay under 64).
+hipError_t linear_mfma_setup() {
+  const void* fns[2] = {(const void*)linear_mfma_kernel<RMOE_FMT_Q4NX, 2, 4, 4>,
+                        (const void*)linear_mfma_kernel<RMOE_FMT_BFP16, 2, 4, 4>};
+  for (const void* f : fns) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)linear_lds(2, 4, 8));
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_linear_mfma(const uint8_t* tiles, int fmt, int M, int K, const uint16_t* x, int T, uint16_t* y,

@@ -381,7 +381,7 @@ int rmoe_create(int device, rmoe_ctx** out) {
   }
   bool ok = hipHostMalloc((void**)&ctx->pinned, kPinnedBytes, hipHostMallocDefault) == hipSuccess &&
             hipHostGetDevicePointer((void**)&ctx->pinned_dev, ctx->pinned, 0) == hipSuccess;
-  ok = ok && rmoe::prefill_setup() == hipSuccess;
+  ok = ok && rmoe::prefill_setup() == hipSuccess && rmoe::linear_mfma_setup() == hipSuccess;
   for (hipEvent_t& ev : ctx->chunk_done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
   if (!ok) {
     free_base(ctx);

@@ -55,6 +55,16 @@ def test_batches_are_stacked_rows(gpu_ctx, fmt, M, K):
 
 
 @pytest.mark.parametrize("fmt", ["q4nx", "bfp16"])
+def test_largest_tile_of_eight_waves(gpu_ctx, fmt):
+    """K = 8,192 (eight waves) with enough tokens for the 32 x 64 tiles: the most LDS of all."""
+    T = 3553
+    mat, w, rng = _matrix(gpu_ctx, fmt, 256, 8192, 11)
+    x = f32_to_bf16(rng.standard_normal((T, 8192), dtype=np.float32))
+    _check(mat.linear(x), x, w)
+    mat.free()
+
+
+@pytest.mark.parametrize("fmt", ["q4nx", "bfp16"])
 @pytest.mark.parametrize("T", [3, 20])
 def test_operands_at_odd_addresses(gpu_ctx, fmt, T):
     """x or y that the 16- and 8-byte accesses cannot take run the K-split kernels."""

@@ -476,7 +476,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
                      bf16x2_to_f16x2(v.w, ex));
     if (r < nrows && c == 0) a.out_exp[(size_t)(row0 + r) * eho + nt] = (int8_t)ex;
   }
-  if (nt == a.n_tiles - 1)
+  if (nt == a.n_tiles - 1 && a.inter < a.out_ld)
     for (int r = tid >> 4; r < nrows; r += 16) zero_row_padding(a, row0 + r, tid & 15, 16);
 }
 

@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const uint32_t* __r
                        bf16x2_to_f16x2(v.w, ex));
       if (r < nrows && c == 0) a.out_exp[(size_t)(row0 + r) * eso + nt] = (int8_t)ex;
     }
-    if (nt == a.n_tiles - 1)
+    if (nt == a.n_tiles - 1 && a.inter < a.out_ld)
       for (int r = tid >> 4; r < nrows; r += 32) zero_row_padding(a, row0 + r, tid & 15, 16);
   } else {
     // Output columns 0..127 of the 256 in slot 0 (fragment 0), 128..255 in slot 1.

@@ -220,7 +220,7 @@ def lm_head_bench(ctx, stream, seed: int, n: int = 50):
     secs = time_graph(g, 1, stream) / n
     mat.free()
     gbs = nbytes / secs / 1e9
-    return {"workload": "lm_head bfp16ebs8 GEMV [260096, 2560], 1 token (linear_bfp16_kernel)",
+    return {"workload": "lm_head bfp16ebs8 GEMV [260096, 2560], 1 token (linear_mfma_kernel)",
             "us_per_launch": round(secs * 1e6, 2), "bytes_per_launch": nbytes, "GBps": round(gbs, 1),
             "frac_hbm_peak": round(gbs / HBM_PEAK_GBS, 4), "traffic": LM_HEAD_TRAFFIC_BYTES}
 
@@ -638,7 +638,7 @@ def profile_pass(ctx, layers, geom, args, stream, gen) -> int:
 
 def _kind_profile_pass(name: str) -> str:
     """Kernel kind of a dispatch of `bench.py --profile-pass`."""
-    return "stack" if "decode_stack" in name else "lm_head" if "linear_bfp16" in name else "copy"
+    return "stack" if "decode_stack" in name else "lm_head" if "linear_mfma" in name else "copy"
 
 
 # Kernel kinds of a dispatch of `bench.py --profile-configs` (the first match counts;
@@ -646,7 +646,7 @@ def _kind_profile_pass(name: str) -> str:
 _CONFIG_KINDS = (("copyBuffer", "copy"), ("CopyBuffer", "copy"), ("linear_lane_kernel", "config1"),
                  ("decode_stack_kernel", "config2"), ("router_prep_kernel", "c3_router"),
                  ("topk_kernel", "c3_topk"), ("dispatch_scatter_kernel", "c3_scatter"),
-                 ("grouped_gemm_kernel", "c3_gemm"), ("h_unify_kernel", "c3_unify"), ("combine_kernel", "c3_combine"))
+                 ("few_rows_gemm_kernel", "c3_gemm"), ("combine_kernel", "c3_combine"))
 
 
 def _kind_profile_configs(name: str) -> str | None:
@@ -737,7 +737,7 @@ def measure_traffic(args) -> dict | None:
         return None
     child = ["--profile-pass", "--no-prefill", "--seed", str(args.seed), "--layers", str(args.layers)] + (
         ["--no-lm-head"] if args.no_lm_head else [])
-    res = _calibrated_passes(child, _kind_profile_pass, "decode_stack|linear_bfp16|copy|Copy", "stack")
+    res = _calibrated_passes(child, _kind_profile_pass, "decode_stack|linear_mfma|copy|Copy", "stack")
     if res is None or "stack" not in res["FETCH_SIZE"] or "stack" not in res["WRITE_SIZE"]:
         return None
     med = {c: {k: statistics.median(v) for k, v in res[c].items()} for c in ("FETCH_SIZE", "WRITE_SIZE")}
@@ -768,7 +768,7 @@ def measure_config_traffic(args) -> dict | None:
     if res is None:
         return None
     out = {}
-    c3_kinds = ("c3_router", "c3_topk", "c3_scatter", "c3_unify", "c3_combine")
+    c3_kinds = ("c3_router", "c3_topk", "c3_scatter", "c3_combine")
     for c in ("FETCH_SIZE", "WRITE_SIZE"):
         r = res[c]
         if not all(k in r for k in ("config1", "config2", "c3_gemm") + c3_kinds) or len(r["c3_gemm"]) < 2:

@@ -108,7 +108,10 @@ int rmoe_matrix_upload_q4k(rmoe_ctx* ctx, const void* q4k_bytes, size_t nbytes, 
 /* y[T, M] = RTNE_bf16(x[T, K] @ W^T), fp32 accumulation.  Replaces NpuBackend.linear /
  * _execute_gemv for a q4nx or bfp16 bundle (npu/backend.py:3569-3721, 3908-4021) and
  * Backend.linear_batch (host/backend.py:71-74).  K_in <= K: columns past K_in are zero
- * padding (comp.padded_k > comp.orig_k, npu/backend.py:3680-3684). */
+ * padding (comp.padded_k > comp.orig_k, npu/backend.py:3680-3684).  rmoe_linear gives a
+ * token the same bytes alone and in a batch; rmoe_linear_dev does so except for T = 1 of a
+ * q4nx matrix with M < 2048 and K = 512, 1024, 2048 or 4096, whose fp32 sums are added in
+ * another order (a faster kernel), so that last bits may differ. */
 int rmoe_linear(rmoe_ctx* ctx, int handle, const uint16_t* x, int T, int K_in, uint16_t* y);
 int rmoe_linear_dev(rmoe_ctx* ctx, int handle, const void* x_dev, int T, void* y_dev, void* stream);
 /* Size the scratch that rmoe_linear_dev needs for up to T tokens on this matrix. */

@@ -11,8 +11,9 @@
 //
 // One workgroup takes 16 MF tokens x 16 NF weight rows, its W waves a W-th of K each; the
 // waves' sums meet in LDS and are added in wave order.  W depends on K only and a row's
-// sums do not depend on MF and NF, so a token's result is the same in a batch of any size
-// (linear_batch equals stacked linear calls).
+// sums do not depend on MF and NF, so a token's result is the same in a batch of any size:
+// linear_batch equals stacked linear calls.  (One token of a small q4nx matrix on device
+// pointers runs linear_lane_kernel instead, whose last bit may differ.)
 #include <algorithm>
 
 #include "wave_gemm.h"

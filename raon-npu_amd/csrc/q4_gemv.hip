@@ -8,7 +8,8 @@
 // write fp32 partials and the last workgroup of a band (device-scope counter) adds
 // them in K order, so the result does not depend on arrival order.
 // It serves the operands that linear_mfma.hip does not take (x or y at an odd address);
-// one token of a small matrix takes linear_lane_kernel.
+// one token of a small matrix takes linear_lane_kernel where the caller does not ask for
+// the bytes of a batch (its sums are in another order).
 #include <algorithm>
 
 #include "../../include/raon_moe.h"
@@ -174,14 +175,14 @@ __global__ __launch_bounds__(64) void linear_lane_kernel(LinearArgs a) {
 
 }  // namespace
 
-hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y, RmoeScratch& s,
-                         hipStream_t st) {
+hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y, bool as_batch,
+                         RmoeScratch& s, hipStream_t st) {
   const int nkt = K / kTileCols, n_rt = M / kTileRows;
   const int ychunks = (T + kNT - 1) / kNT;
   // One token of a small matrix (fewer than 32 row bands) with 4..32 K tiles: one wave
   // per workgroup, two lanes per K tile of a row (config 1: 3.05 -> 2.07 us per launch in
   // a graph against one lane per K tile with x staged in LDS; the MFMA kernel takes 3.6 us).
-  if (T == 1 && n_rt < 32 && (nkt == 4 || nkt == 8 || nkt == 16 || nkt == 32) &&
+  if (T == 1 && !as_batch && n_rt < 32 && (nkt == 4 || nkt == 8 || nkt == 16 || nkt == 32) &&
       (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     LinearArgs a{tiles, M, K, x, T, y, nullptr, nullptr, 1};
     const dim3 grid(M / (32 / nkt)), block(64);

@@ -434,8 +434,10 @@ hipError_t launch_quantize(const float* w, int M, int K, int ld, int k_valid, ui
 hipError_t launch_synth_quantize(uint64_t seed, float std, int M, int K, int k_valid, uint8_t* tiles, int* err,
                                  hipStream_t st);
 
-hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y, RmoeScratch& s,
-                         hipStream_t st);
+// as_batch: one token gets the bytes it has in a batch (the order of linear_mfma.hip);
+// otherwise one token of a small matrix takes the faster linear_lane_kernel.
+hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y, bool as_batch,
+                         RmoeScratch& s, hipStream_t st);
 
 // Both formats on MFMA (linear_mfma.hip), for the operands linear_mfma_ok() accepts.
 bool linear_mfma_ok(int M, int K, const uint16_t* x, int T, const uint16_t* y);

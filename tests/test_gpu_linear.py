@@ -26,6 +26,18 @@ def _case(M, K, seed, std=0.02):
     return pack_gemv(c, s, m), dequantize_simple(c, s, m), rng
 
 
+def _linear_dev(mat, x):
+    """``linear`` on device pointers, which runs linear_lane_kernel for one token of a small matrix."""
+    import torch
+
+    xd = torch.from_numpy(x.view(np.int16)).cuda()
+    yd = torch.empty(x.shape[0], mat.M, dtype=torch.int16, device="cuda")
+    mat.reserve(x.shape[0])
+    mat.linear_dev(xd, x.shape[0], yd, stream=torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    return yd.cpu().numpy().view(np.uint16)
+
+
 def test_config1_gemv(gpu_ctx):
     # BASELINE config 1: W 768x2048 N(0,0.02), x 1x2048 bf16 N(0,1), seed 0.
     blob, wf, _ = _case(768, 2048, 0)
@@ -41,8 +53,7 @@ def test_config1_gemv(gpu_ctx):
 
 
 @pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 9])
-# K <= 4096 runs one workgroup per row band (linear_band_kernel); K = 5120 runs the K-split
-# kernel with its partials and ordered final sum.
+# 2 to 40 K tiles, the latter over four waves of 10.
 @pytest.mark.parametrize("M,K", [(128, 256), (1536, 2048), (2048, 768), (2176, 2560), (256, 5120)])
 def test_gemv_tokens_and_shapes(gpu_ctx, T, M, K):
     blob, wf, rng = _case(M, K, M * 7 + K + T)
@@ -95,13 +106,14 @@ def test_gemv_extreme_inputs(gpu_ctx):
 
 
 # One token of a matrix with fewer than 32 row bands and 4, 8, 16 or 32 K tiles runs
-# linear_lane_kernel (two lanes per K tile, x straight from memory, group sums on v_dot2).
+# linear_lane_kernel on device pointers (two lanes per K tile, x straight from memory, group
+# sums on v_dot2).
 @pytest.mark.parametrize("M,K", [(128, 512), (256, 1024), (128, 4096), (1920, 2048), (384, 2048)])
 def test_gemv_single_token_lane_kernel(gpu_ctx, M, K):
     blob, wf, rng = _case(M, K, M * 11 + K)
     x = f32_to_bf16(rng.standard_normal((1, K)).astype(np.float32))
     mat = gpu_ctx.upload_matrix(blob, M, K)
-    y = mat.linear(x)
+    y = _linear_dev(mat, x)
     ref = om.linear(wf, x[0])[None]
     err, rel, same = compare_bf16(y, ref)
     assert err <= 1e-2 and rel <= 1e-3 and same >= 0.99, (err, rel, same)
@@ -124,7 +136,7 @@ def test_gemv_single_token_extreme_inputs(gpu_ctx):
     alt[1::2] = f32_to_bf16(-np.ones(K // 2, np.float32))
     rows.append(alt)
     for t, xr in enumerate(rows):
-        y = mat.linear(xr[None])[0]
+        y = _linear_dev(mat, xr[None])[0]
         ref = om.linear(wf, xr)
         if t == 0:
             assert np.all(y == 0)

@@ -16,7 +16,8 @@ from oracle.q4nx import dequantize_simple, pack_gemv, quantize
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(128, 256), (384, 768), (2176, 2560), (128, 12032)]
+# (128, 512) and (768, 2048) in q4nx are shapes whose one-token device calls run the GEMV.
+SHAPES = [(128, 256), (384, 768), (2176, 2560), (128, 12032), (128, 512), (768, 2048)]
 
 
 def _matrix(gpu_ctx, fmt, M, K, seed):
@@ -39,18 +40,16 @@ def _check(y, x, w):
 @pytest.mark.parametrize("fmt", ["q4nx", "bfp16"])
 @pytest.mark.parametrize("M,K", SHAPES)
 def test_batches_are_stacked_rows(gpu_ctx, fmt, M, K):
-    """Every batch size against float64, and a row's bytes the same in all of them (one row
-    of a small q4nx matrix runs the GEMV and is only held to the bound)."""
+    """Every batch size against float64, and a row's bytes the same in all of them, a batch
+    of one row included."""
     mat, w, rng = _matrix(gpu_ctx, fmt, M, K, M + 3 * K)
     x = f32_to_bf16(rng.standard_normal((70, K)).astype(np.float32))
     full = mat.linear(x)
     _check(full, x, w)
-    for T in (1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 64, 65):
-        y = mat.linear(x[:T])
-        if T == 1 and fmt == "q4nx":
-            _check(y, x[:1], w)
-        else:
-            np.testing.assert_array_equal(y, full[:T], err_msg=f"T={T}")
+    for T in (2, 4, 5, 15, 16, 17, 31, 32, 33, 64, 65):
+        np.testing.assert_array_equal(mat.linear(x[:T]), full[:T], err_msg=f"T={T}")
+    for t in range(70):
+        np.testing.assert_array_equal(mat.linear(x[t:t + 1])[0], full[t], err_msg=f"row {t} alone")
     mat.free()
 
 

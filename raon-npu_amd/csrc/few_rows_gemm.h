@@ -11,8 +11,9 @@
 // resident per CU, each hiding the other's prologue and load rounds.
 // Of a weight tile's 5 KB, 1 KB are scales and mins, which the correction needs before the K
 // loop: their scales stay in LDS from there on (2 KB per K tile, 32 to 40 KB per workgroup;
-// reading them again beside the codes cost 3 to 7 % of gate/up), and the first block of them
-// is requested with the first codes, before the row indices are known.
+// reading them again beside the codes cost 3 to 7 % of gate/up) as long as two workgroups fit
+// a CU, and the first block of them is requested with the first codes, before the row indices
+// are known.
 // Kernel times against grouped_gemm_kernel, gate/up and down: H=2048, I=768, 445 tokens 95 ->
 // 80 and 57 -> 47 us; H=2560, I=1088, 32 tokens 108 -> 79 and 61 -> 44 us, 256 tokens 142 ->
 // 119 and (bfp16) 139 -> 104 us: 4.2 to 4.9 TB/s of expert weights over the whole kernel.  The
@@ -31,7 +32,8 @@ constexpr int kFewDownOut = kBMFew * 264 * 2;
 
 // One tile of 16 MF rows by 256 weight rows.  Gate/up: units 128 nt + 32 w .. +31 in wave w
 // (fragments 0, 1 gate, 2, 3 up); down: output columns 256 nt + 64 w .. +63.
-template <int MF, bool kDown, bool kB16>
+// kWide: the scales of a K tile come with its codes instead of from LDS (few_rows_wide).
+template <int MF, bool kDown, bool kB16, bool kWide>
 __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, int nt, uint8_t* lds, int* rowidx,
                                               int8_t* row_e, int* differ) {
   constexpr int NF = 4;
@@ -56,12 +58,13 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     if (dead) wrow[f] = 0;
     wf[f] = W + (size_t)(wrow[f] / kTileRows) * wkt * kTB + (wrow[f] % kTileRows) * 16;
   }
-  // Weights of one K tile.  q4nx: codes of (row l16, group lq), the scales come from LDS;
+  // Weights of one K tile.  q4nx: codes of (row l16, group lq), the scales come from LDS or,
+  // kWide, the group's scale | min word;
   // bfp16: mantissas of columns 32 lq .. +31 and their four exponents.  The first two tiles
   // depend on the tile entry only: requested before anything else.
   struct WTile {
     uint4 c[NF][kB16 ? 2 : 1];
-    uint32_t s[kB16 ? NF : 1];
+    uint32_t s[kB16 || kWide ? NF : 1];
   };
   auto load_w = [&](int kt, WTile& w) {
     const bool live = kt < nkt && !dead;
@@ -74,6 +77,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
         w.s[f] = wg_load<uint32_t>(p + kB16MantBytes, live ? 16u * l16 + 4u * lq : 0u);
       } else {
         w.c[f][0] = wg_load_weights<true>(p, live ? 1024u * lq + 16u * l16 : 0u);
+        if constexpr (kWide) w.s[f] = wg_load<uint32_t>(p + kCodeBytes, live ? 16u * l16 + 4u * lq : 0u);
       }
     }
     asm volatile("" ::: "memory");  // keeps the loads where they are
@@ -150,7 +154,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
   if constexpr (!kB16) load_s(0, sa);
   // What is in flight during the correction, as far as registers go (a spill is never worth
   // it here: one has corrupted row addresses).  256 registers with these, none spilled.
-  constexpr bool kCoefAhead = MF <= 2, kSumsAhead = MF <= 1, kRowsAhead = MF <= 1;
+  constexpr bool kCoefAhead = MF <= (kWide ? 1 : 2), kSumsAhead = MF <= 1, kRowsAhead = MF <= 1;
   if constexpr (kRowsAhead) {
     load_x(0);
     asm volatile("" ::: "memory");
@@ -216,7 +220,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     for (int f = 0; f < NF; ++f) acc[m][f] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // The wave's scales, for the K loop: [K tile][fragment][row][group] bf16 in LDS.
-  uint8_t* wsc = lds + kFewStageBytes + (size_t)wave * wkt * (NF * 128) + 8 * l16;
+  [[maybe_unused]] uint8_t* wsc = lds + kFewStageBytes + (size_t)wave * wkt * (NF * 128) + 8 * l16;
   int fx[NF];
   [[maybe_unused]] int emax_w[NF];
   {
@@ -238,7 +242,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
                                   b.c[f][1].x, b.c[f][1].y, b.c[f][1].z, b.c[f][1].w};
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            if (gl + 4 * h < G)
+            if (!kWide && gl + 4 * h < G)
               *reinterpret_cast<uint2*>(wsc + ((8 * blk + 2 * lq + h) * NF + f) * 128) =
                   make_uint2(__builtin_amdgcn_perm(sv[4 * h + 1], sv[4 * h], 0x05040100u),
                              __builtin_amdgcn_perm(sv[4 * h + 3], sv[4 * h + 2], 0x05040100u));
@@ -332,7 +336,9 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
       if constexpr (!kB16) {
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
-          const float sc = bf16_to_f32(*reinterpret_cast<const uint16_t*>(wsc + (kt * NF + f) * 128 + 2 * lq));
+          float sc;
+          if constexpr (kWide) sc = bf16_to_f32(w.s[f] & 0xffffu);
+          else sc = bf16_to_f32(*reinterpret_cast<const uint16_t*>(wsc + (kt * NF + f) * 128 + 2 * lq));
           const float v1 = __builtin_amdgcn_ldexpf(sc, -fx[f]), v16 = __builtin_amdgcn_ldexpf(sc, -fx[f] - 4);
           s1[f] = __builtin_bit_cast(f16x2_t, __builtin_amdgcn_cvt_pkrtz(v1, v1));
           s16[f] = __builtin_bit_cast(f16x2_t, __builtin_amdgcn_cvt_pkrtz(v16, v16));
@@ -481,15 +487,23 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
 }
 
 // Dynamic LDS: the stages and, with q4nx weights, the four waves' scales (2 KB per K tile);
-// then, in the same place, the epilogue staging.
+// then, in the same place, the epilogue staging.  Two workgroups of it share a CU's 160 KB
+// (with 1 KB for what the kernel declares itself): a layer whose scales take more than that
+// (K over 3,328) reads them beside the codes instead, at any width.  With one workgroup per CU
+// whole layers of 32 experts took, against this form: H = 4096, I = 768, 368 tokens 138.5 /
+// 116.6 us, H = I = 4096, 256 tokens 374 / 307 us; batches that fill less than one workgroup per
+// CU lose 2 to 6 % by it (H = 3584, I = 768, 32 tokens 65.9 / 70.0 us).
+constexpr size_t kFewMaxLds = (size_t)79 << 10;
+constexpr size_t few_rows_scales(int K) { return (size_t)4 * (K / kTileCols) * 512; }
+constexpr bool few_rows_wide(int K, bool b16) { return !b16 && kFewStageBytes + few_rows_scales(K) > kFewMaxLds; }
 static size_t few_rows_lds(const GemmArgs& a, bool b16) {
-  const size_t loop = kFewStageBytes + (b16 ? 0 : (size_t)4 * (a.K / kTileCols) * 512);
+  const size_t loop = kFewStageBytes + (b16 || few_rows_wide(a.K, b16) ? 0 : few_rows_scales(a.K));
   return std::max(loop, (size_t)(a.mode == 0 ? kFewGateUpOut : kFewDownOut));
 }
 
 // Grid: as grouped_gemm_kernel's, 256 threads.  XCD x takes a contiguous eighth of each
 // class's tiles, the largest first.
-template <bool kDown, bool kB16>
+template <bool kDown, bool kB16, bool kWide>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void few_rows_gemm_kernel(GemmArgs a, int cap) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // few_rows_lds() bytes
   __shared__ int rowidx[kBMFew];
@@ -509,9 +523,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t te = a.tiles[(size_t)c * cap + lid / a.n_tiles];
     const int nt = lid % a.n_tiles;
     if (skip_tile(a, te)) return;
-    if (c == 2) few_rows_tile<3, kDown, kB16>(a, te, nt, lds, rowidx, row_e, &differ);
-    else if (c == 1) few_rows_tile<2, kDown, kB16>(a, te, nt, lds, rowidx, row_e, &differ);
-    else few_rows_tile<1, kDown, kB16>(a, te, nt, lds, rowidx, row_e, &differ);
+    if (c == 2) few_rows_tile<3, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);
+    else if (c == 1) few_rows_tile<2, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);
+    else few_rows_tile<1, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);
     return;
   }
 }

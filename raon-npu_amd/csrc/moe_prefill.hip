@@ -1593,9 +1593,11 @@ static hipError_t launch_grouped(GemmArgs a, uint32_t* tiles, int* ntiles, int c
   if (few) {
     const dim3 grid(per2 + 2 * per01), block(256);
     const size_t lds = few_rows_lds(a, b16);
-    auto* kernel = a.mode == 0 ? few_rows_gemm_kernel<false, false>
-                   : b16       ? few_rows_gemm_kernel<true, true>
-                               : few_rows_gemm_kernel<true, false>;
+    const bool wide = few_rows_wide(a.K, b16);
+    auto* kernel = a.mode == 0 ? (wide ? few_rows_gemm_kernel<false, false, true> : few_rows_gemm_kernel<false, false, false>)
+                   : b16       ? few_rows_gemm_kernel<true, true, false>
+                   : wide      ? few_rows_gemm_kernel<true, false, true>
+                               : few_rows_gemm_kernel<true, false, false>;
     hipLaunchKernelGGL(kernel, grid, block, lds, st, a, cap);
   } else if (b16) {
     hipLaunchKernelGGL((grouped_gemm_kernel<7, true>), dim3(per2 + 2 * per01), dim3(512), 0, st, a, cap);
@@ -1605,13 +1607,12 @@ static hipError_t launch_grouped(GemmArgs a, uint32_t* tiles, int* ntiles, int c
   return hipGetLastError();
 }
 
-// Allow the few-rows kernels the dynamic LDS of the widest layer (K = 8192).
+// Allow the few-rows kernels with scales in LDS the most they ask for (the others stay under 64 KB).
 hipError_t prefill_setup() {
-  const int lds = kFewStageBytes + 4 * (8192 / kTileCols) * 512;
-  const void* fns[3] = {(const void*)few_rows_gemm_kernel<false, false>, (const void*)few_rows_gemm_kernel<true, true>,
-                        (const void*)few_rows_gemm_kernel<true, false>};
+  const void* fns[2] = {(const void*)few_rows_gemm_kernel<false, false, false>,
+                        (const void*)few_rows_gemm_kernel<true, false, false>};
   for (const void* f : fns) {
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFewMaxLds);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1624,11 +1625,14 @@ hipError_t prefill_setup() {
 // 200, 1,024 248 / 236; H=2560, I=1088, 6 of 128: 300 tokens 214 / 259, 1,000 (47 rows) 346 /
 // 358, 2,000 576 / 560.
 constexpr int kFewRows = 46;
-static bool few_rows(size_t assignments, int n_routed) { return assignments <= (size_t)kFewRows * n_routed; }
+static bool few_rows(const RmoeLayer& L, int T) {
+  const size_t A = (size_t)T * L.top_k;
+  return A <= (size_t)kFewRows * L.n_routed && (A + T) * L.Ipad * 2 < (size_t)1 << 32;  // byte offsets into h
+}
 // Tiles of a class at most: the full ones and one remainder per group.
 static size_t tile_capacity(const RmoeLayer& L, int T) {
   const size_t A = (size_t)T * L.top_k;
-  const int bm = few_rows(A, L.n_routed) ? kBMFew : kBM;
+  const int bm = few_rows(L, T) ? kBMFew : kBM;
   return A / bm + L.n_routed + T / bm + 4;
 }
 
@@ -1675,7 +1679,7 @@ hipError_t launch_moe_prefill(const RmoeLayer& L, const uint16_t* x, int T, cons
   int8_t* xexp = (int8_t*)carve((size_t)T);
   uint16_t* xsum = (uint16_t*)carve((size_t)T * 3 * Gpx * 2);
   float* logits = (float*)carve((size_t)T * E * 16);
-  const bool few = few_rows(A, E);
+  const bool few = few_rows(L, T);
   const int bm = few ? kBMFew : kBM, tile_cap = (int)tile_capacity(L, T);
   uint32_t* tiles = (uint32_t*)carve((size_t)kTileClasses * tile_cap * 4);
   int* ntiles = (int*)carve(256);

@@ -13,8 +13,9 @@ import pytest
 
 from raon_npu_amd import geometry as G
 
-from moe_fixtures import make_layer, random_tokens
+from moe_fixtures import compare_bf16, make_layer, random_tokens
 from oracle import bfp16 as B
+from oracle import moe as om
 
 pytestmark = pytest.mark.gpu
 
@@ -28,8 +29,8 @@ def _routes(rng, T):
     return np.stack([rng.choice(16, 2, replace=False, p=p / p.sum()) for _ in range(T)]).astype(np.int32)
 
 
-def _tokens(T, seed):
-    x = random_tokens(T, 512, seed)
+def _tokens(T, seed, hidden=512):
+    x = random_tokens(T, hidden, seed)
     u = x.astype(np.uint32)
     # rows 5, 25, 45, ...: a hundred times 2^12 larger, rows 6, 26, ... 2^-14 smaller
     for r0, shift in ((5, 12), (6, -14)):
@@ -88,21 +89,28 @@ def test_few_rows_prefill_equals_many_rows(gpu_ctx):
     lyr.free()
 
 
-# Blocks of 32 groups in the correction: one, two and a quarter, three and a quarter, eight (the
-# widest layer, whose scales fill LDS); rows per group for each tile class.
-@pytest.mark.parametrize("hidden", [1024, 2304, 3328, 8192])
-def test_few_rows_widths(gpu_ctx, hidden):
-    geom = G.MoeGeometry(hidden=hidden, inter=64, n_routed=4, n_shared=1, top_k=1)
+# Blocks of 32 groups in the correction: one, two and a quarter, three and a quarter (the widest
+# whose scales stay in LDS), three and a half, eight; the same for the down GEMM, whose width is
+# not limited (8,704: with its scales in LDS a workgroup would take more than a CU has); rows per
+# group for each tile class.
+@pytest.mark.parametrize("hidden,inter", [(1024, 64), (2304, 64), (3328, 64), (3584, 64), (8192, 64), (256, 3328),
+                                          (256, 3392), (256, 8704)])
+def test_few_rows_widths(gpu_ctx, hidden, inter):
+    geom = G.MoeGeometry(hidden=hidden, inter=inter, n_routed=4, n_shared=1, top_k=1)
     syn = make_layer(geom, seed=77)
     lyr = gpu_ctx.create_layer(1702, geom)
     lyr.upload_experts(syn.gate_up, syn.down)
-    x = random_tokens(260, hidden, 78)
+    x = _tokens(260, 78, hidden)
     ids = np.repeat(np.arange(4), [5, 16, 30, 209]).astype(np.int32)[:, None]
     wts = np.ones(ids.shape, np.float32)
-    sgu = random_tokens(260, 128, 79)
+    sgu = random_tokens(260, 2 * inter, 79)
     want_r, want_s = lyr.moe_experts_grouped(x, ids, wts, sgu)  # 65 rows per expert: the general kernel
     for T in (5, 51, 98):  # the last groups hold 5, 30 and 47 rows
         r, s = lyr.moe_experts_grouped(x[:T], ids[:T], wts[:T], sgu[:T])
         np.testing.assert_array_equal(r, want_r[:T], err_msg=f"routed, T={T}")
         np.testing.assert_array_equal(s, want_s[:T], err_msg=f"shared, T={T}")
+    bank = syn.bank()
+    for t in (0, 21, 97):
+        _, rel, _ = compare_bf16(want_r[t], om.moe_experts(bank, x[t], ids[t], wts[t], 4.0, 25.0))
+        assert rel <= 4e-3, (t, rel)  # one bf16 rounding per element: 2^-8
     lyr.free()

@@ -153,7 +153,8 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
   };
   if constexpr (!kB16) load_s(0, sa);
   // What is in flight during the correction, as far as registers go (a spill is never worth
-  // it here: one has corrupted row addresses).  256 registers with these, none spilled.
+  // it here: the compiler has placed one so that it corrupted row addresses).  236 to 243 of
+  // 256 registers with these.
   constexpr bool kCoefAhead = MF <= (kWide ? 1 : 2), kSumsAhead = MF <= 1, kRowsAhead = MF <= 1;
   if constexpr (kRowsAhead) {
     load_x(0);
@@ -387,6 +388,12 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
   }
   __syncthreads();  // every wave is past its activation region: LDS becomes the output staging
 
+  // The thread's place as a value of its own from here on: derived from tid, the epilogue's
+  // indices are the same in the three tile sizes, and the compiler computes them once at the
+  // kernel's start and holds them in some ten registers through the K loop.
+  int et = tid;
+  asm volatile("" : "+v"(et));
+  const int el16 = et & 15, elq = (et >> 4) & 3;
   uint16_t* stage = reinterpret_cast<uint16_t*>(lds);
   if constexpr (kDown) {
     // [16 MF rows][256 columns + 8]
@@ -398,12 +405,12 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
           const uint32_t p2 = cvt_bf16x2(acc[m][f][i], acc[m][f][i + 1]);
-          uint16_t* st = stage + (16 * m + 4 * lq + i) * kStride + 64 * wave + 16 * f + l16;
+          uint16_t* st = stage + (16 * m + 4 * elq + i) * kStride + 64 * wave + 16 * f + el16;
           st[0] = (uint16_t)(p2 & 0xffffu);
           st[kStride] = (uint16_t)(p2 >> 16);
         }
     __syncthreads();
-    for (int cid = tid; cid < nrows * 32; cid += 256) {
+    for (int cid = et; cid < nrows * 32; cid += 256) {
       const int r = cid >> 5, c = cid & 31;
       *reinterpret_cast<uint4*>(a.out + (size_t)(row0 + r) * a.out_ld + 256 * nt + 8 * c) =
           *reinterpret_cast<const uint4*>(stage + r * kStride + 8 * c);
@@ -425,7 +432,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
             const float h0 = swiglu_fast(bf16_to_f32(gu0 & 0xffffu), __uint_as_float(gu0 & 0xffff0000u));
             const float h1 = swiglu_fast(bf16_to_f32(gu1 & 0xffffu), __uint_as_float(gu1 & 0xffff0000u));
             const uint32_t hp = cvt_bf16x2(h0, h1);
-            uint16_t* st = stage + (16 * m + 4 * lq + i) * kOutStride + 32 * wave + 16 * q + l16;
+            uint16_t* st = stage + (16 * m + 4 * elq + i) * kOutStride + 32 * wave + 16 * q + el16;
             st[0] = (uint16_t)(hp & 0xffffu);
             st[kOutStride] = (uint16_t)(hp >> 16);
           }
@@ -437,7 +444,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const uint32_t gu = cvt_bf16x2(acc[m][q][i], acc[m][q + 2][i]);
-            const int at = (16 * m + 4 * lq + i) * kOutStride + 32 * wave + 16 * q + l16;
+            const int at = (16 * m + 4 * elq + i) * kOutStride + 32 * wave + 16 * q + el16;
             stage[rows_b + at] = (uint16_t)(gu & 0xffffu);
             stage[2 * rows_b + at] = (uint16_t)(gu >> 16);
           }
@@ -446,7 +453,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
   __syncthreads();
   const int units = min(128, a.inter - 128 * nt);  // live units of the tile (a multiple of 64)
   if (a.act != 1) {
-    for (int idx = tid; idx < nrows * 128; idx += 256) {
+    for (int idx = et; idx < nrows * 128; idx += 256) {
       if ((idx & 127) >= units) continue;
       const int at = (idx >> 7) * kOutStride + (idx & 127);
       stage[at] = (uint16_t)cvt_bf16x2(
@@ -455,8 +462,8 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     __syncthreads();
   }
   const int Gpo = sum_planes_gp(a.out_ld / 32), eho = exp_stride(a.out_ld);
-  if (tid < 64 * MF) {
-    const int r = tid >> 2, q = tid & 3;
+  if (et < 64 * MF) {
+    const int r = et >> 2, q = et & 3;
     if (r < nrows && 32 * q < units) {
       float hs = 0.f;
 #pragma unroll
@@ -471,7 +478,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
   }
 #pragma unroll
   for (int q = 0; q < MF; ++q) {
-    const int cid = tid + 256 * q, r = cid >> 4, c = cid & 15;
+    const int cid = et + 256 * q, r = cid >> 4, c = cid & 15;
     const bool live = 8 * c < units;
     const uint4 v = *reinterpret_cast<const uint4*>(stage + r * kOutStride + 8 * c);
     const float mx = row16_max(live ? max_abs_bf16x8(v) : 0.f);
@@ -483,7 +490,7 @@ __device__ __forceinline__ void few_rows_tile(const GemmArgs& a, uint32_t te, in
     if (r < nrows && c == 0) a.out_exp[(size_t)(row0 + r) * eho + nt] = (int8_t)ex;
   }
   if (nt == a.n_tiles - 1 && a.inter < a.out_ld)
-    for (int r = tid >> 4; r < nrows; r += 16) zero_row_padding(a, row0 + r, tid & 15, 16);
+    for (int r = et >> 4; r < nrows; r += 16) zero_row_padding(a, row0 + r, et & 15, 16);
 }
 
 // Dynamic LDS: the stages and, with q4nx weights, the four waves' scales (2 KB per K tile);

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -32,6 +33,8 @@ COMMON = [
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# Prints each kernel's registers, spills and scratch memory for check_spills().
+REPORT = "-Rpass-analysis=kernel-resource-usage"
 
 
 def hipcc() -> str:
@@ -41,13 +44,33 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the HIP toolchain is required to build librmoe.so")
 
 
+def check_spills(src: Path, report: str) -> None:
+    """Refuse an object whose kernels spill vector registers (``report``: the compiler's
+    resource remarks).  In a kernel at its register limit the compiler has placed spills
+    where only part of the lanes were saved, so that the others reloaded stale row
+    addresses; such an object must not reach a GPU, whichever compiler version made it."""
+    kernels = re.split(r"remark:\s+Function Name: ", report)[1:]
+    if not kernels and "__global__" in src.read_text():
+        raise RuntimeError(f"{src.name}: the compiler reported no kernel's registers; spills cannot be ruled out")
+    for k in kernels:
+        spills = re.search(r"remark:\s+VGPRs Spill: (\d+)", k)
+        if spills is None or int(spills.group(1)):
+            raise RuntimeError(f"{src.name}: {k.split()[0]} spills vector registers "
+                               f"({spills.group(1) if spills else 'count not reported'})")
+
+
 def _compile(src: Path, build_dir: Path = BUILD, defines: tuple[str, ...] = ()) -> Path:
     obj = build_dir / (src.stem + ".o")
-    cmd = [hipcc(), *COMMON, *(f"-D{d}" for d in defines), "-I", str(PKG.parent / "include"), "-c", str(src),
+    cmd = [hipcc(), *COMMON, REPORT, *(f"-D{d}" for d in defines), "-I", str(PKG.parent / "include"), "-c", str(src),
            "-o", str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{res.stdout}\n{res.stderr}")
+    try:
+        check_spills(src, res.stderr)
+    except RuntimeError:
+        obj.unlink(missing_ok=True)
+        raise
     return obj
 
 

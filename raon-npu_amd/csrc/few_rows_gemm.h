@@ -529,7 +529,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (lid >= n) return;
     const uint32_t te = a.tiles[(size_t)c * cap + lid / a.n_tiles];
     const int nt = lid % a.n_tiles;
-    if (skip_tile(a, te)) return;
     if (c == 2) few_rows_tile<3, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);
     else if (c == 1) few_rows_tile<2, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);
     else few_rows_tile<1, kDown, kB16, kWide>(a, te, nt, lds, rowidx, row_e, &differ);

@@ -256,7 +256,8 @@ __device__ __forceinline__ bool arrive_last(unsigned* counter, unsigned n, unsig
 // that hold rows, so that a group's short last tile does no MFMA work on absent rows.
 //   bm = kBM (128): class 0 (up to 32 rows: 2 fragments), 1 (up to 64: 4), 2 (8);
 //   bm = kBMFew (48): class 0 (up to 16 rows: 1 fragment), 1 (up to 32: 2), 2 (3).
-// Class c's tiles sit at tiles[c * cap ...] in group order, their count in ntiles[c].  A
+// Class c's tiles sit at tiles[c * cap ...] in group order, their count in ntiles[c], the
+// count without the last group's (the shared expert's) in ntiles[kTileClasses + c].  A
 // 48-row tile also carries its row count (few_tile), one dependent read fewer at its start.
 constexpr int kBM = 128;
 constexpr int kBMFew = 48;
@@ -322,6 +323,10 @@ __device__ __forceinline__ void tile_table_block(int e, int ng, int b, int end, 
   for (int c = 0; c < 2; ++c)
     if (cnt[c] && base[c] < cap) tiles[c * cap + base[c]] = entry(b + full * bm);
   if (e < kTileClasses) ntiles[e] = min(e == 0 ? total[0] : e == 1 ? total[1] : total[2], cap);
+  if (e == ng - 1) {
+#pragma unroll
+    for (int c = 0; c < kTileClasses; ++c) ntiles[kTileClasses + c] = min(base[c], cap);
+  }
 }
 
 // Wave-wide (64 lanes) sum.

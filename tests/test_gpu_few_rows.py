@@ -114,3 +114,29 @@ def test_few_rows_widths(gpu_ctx, hidden, inter):
         _, rel, _ = compare_bf16(want_r[t], om.moe_experts(bank, x[t], ids[t], wts[t], 4.0, 25.0))
         assert rel <= 4e-3, (t, rel)  # one bf16 rounding per element: 2^-8
     lyr.free()
+
+
+# The shared group's last tile in each class (12, 32 and 47 rows of 48; 24, 60 and 100 of 128), which
+# the gate/up GEMM leaves out of its tiles: 16 experts (table by the scatter launch), 256 (its own).
+@pytest.mark.parametrize("experts", [16, 256])
+def test_shared_tiles_left_out_of_gate_up(gpu_ctx, experts):
+    geom = G.MoeGeometry(hidden=256, inter=64, n_routed=experts, n_shared=1, top_k=1)
+    syn = make_layer(geom, seed=91)
+    lyr = gpu_ctx.create_layer(1703, geom)
+    lyr.upload_experts(syn.gate_up, syn.down)
+    few, many = (300, 320, 335), tuple(128 * (experts // 2) + r for r in (24, 60, 100))
+    T = max(many)
+    rng = np.random.default_rng(92)
+    x, ids = random_tokens(T, 256, 93), rng.integers(0, experts, (T, 1)).astype(np.int32)
+    wts = np.ones(ids.shape, np.float32)
+    sgu = random_tokens(T, 128, 94)
+    want_r, want_s = lyr.moe_experts_grouped(x, ids, wts, sgu)
+    bank = syn.bank()
+    for t in (0, 150, T - 1):
+        _, rel, _ = compare_bf16(want_r[t], om.moe_experts(bank, x[t], ids[t], wts[t], 4.0, 25.0))
+        assert rel <= 4e-3, (t, rel)  # one bf16 rounding per element: 2^-8
+    for n in few + many:
+        r, s = lyr.moe_experts_grouped(x[:n], ids[:n], wts[:n], sgu[:n])
+        np.testing.assert_array_equal(r, want_r[:n], err_msg=f"routed, T={n}")
+        np.testing.assert_array_equal(s, want_s[:n], err_msg=f"shared, T={n}")
+    lyr.free()

@@ -7,7 +7,7 @@
 // to four waves covers one 64-row band over a range of K tiles; bands split over K
 // write fp32 partials and the last workgroup of a band (device-scope counter) adds
 // them in K order, so the result does not depend on arrival order.
-// It serves the operands that linear_mfma.hip does not take (x or y at an odd address);
+// It serves the operands that linear_mfma.hip does not take (x not 16-byte aligned);
 // one token of a small matrix takes linear_lane_kernel where the caller does not ask for
 // the bytes of a batch (its sums are in another order).
 #include <algorithm>
@@ -192,8 +192,8 @@ hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, 
     else hipLaunchKernelGGL(linear_lane_kernel<32>, grid, block, 0, st, a);
     return hipGetLastError();
   }
-  if (linear_mfma_ok(M, K, x, T, y)) return launch_linear_mfma(tiles, RMOE_FMT_Q4NX, M, K, x, T, y, st);
-  // The other operands (x or y at an address the MFMA kernel cannot load or store from).
+  if (linear_mfma_ok(M, K, x, T)) return launch_linear_mfma(tiles, RMOE_FMT_Q4NX, M, K, x, T, y, st);
+  // The other operands (x at an address the MFMA kernel cannot load from).
   // Up to 4 K tiles per workgroup (one per wave); tall matrices, whose row bands alone
   // fill the chip, split K less (down to one workgroup per band) and skip the partials.
   int ksplit = std::min((nkt + 3) / 4, (kFillGroups + n_rt - 1) / n_rt);

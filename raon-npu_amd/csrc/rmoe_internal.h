@@ -445,7 +445,7 @@ hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, 
                          RmoeScratch& s, hipStream_t st);
 
 // Both formats on MFMA (linear_mfma.hip), for the operands linear_mfma_ok() accepts.
-bool linear_mfma_ok(int M, int K, const uint16_t* x, int T, const uint16_t* y);
+bool linear_mfma_ok(int M, int K, const uint16_t* x, int T);
 hipError_t linear_mfma_setup();  // once per device before the first call
 hipError_t launch_linear_mfma(const uint8_t* tiles, int fmt, int M, int K, const uint16_t* x, int T, uint16_t* y,
                               hipStream_t st);

@@ -251,7 +251,7 @@ hipError_t launch_b16_relayout_out(const uint8_t* tiles, uint8_t* packed, int M,
 
 hipError_t launch_linear_bfp16(const uint8_t* tiles, int M, int K, const uint16_t* x, int T, uint16_t* y,
                                RmoeScratch& s, hipStream_t st) {
-  if (linear_mfma_ok(M, K, x, T)) return launch_linear_mfma(tiles, RMOE_FMT_BFP16, M, K, x, T, y, st);
+  if (linear_mfma_ok(x)) return launch_linear_mfma(tiles, RMOE_FMT_BFP16, M, K, x, T, y, st);
   // The other operands (x at an address the MFMA kernel cannot load from).
   const int nkt = K / kTileCols, n_rt = M / kTileRows;
   const int ksplit = bfp16_ksplit(M, K);

@@ -155,11 +155,8 @@ hipError_t pick(const LinMfmaArgs& a, hipStream_t st) {
 
 }  // namespace
 
-bool linear_mfma_ok(int M, int K, const uint16_t* x, int T) {
-  // 16-byte loads of x rows, 32-bit byte offsets into x, and a grid that fits its counter.
-  return (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-         (size_t)T * K * 2 < ((size_t)1 << 32) && ((size_t)T + 15) / 16 * (M / 16) < ((size_t)1 << 28);
-}
+// 16-byte loads of x rows.
+bool linear_mfma_ok(const uint16_t* x) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0; }
 
 // Allow the 32 x 64 tiles of eight waves their 68 KB of dynamic LDS (the others stay under 64).
 hipError_t linear_mfma_setup() {
@@ -174,10 +171,21 @@ hipError_t linear_mfma_setup() {
   return hipSuccess;
 }
 
+static_assert((size_t)linear_mfma_max_tokens(65536, 512) / 32 * (65536 / 64) * 256 < ((size_t)1 << 32) &&
+                  (size_t)linear_mfma_max_tokens(1 << 22, 8192) / 32 * ((1 << 22) / 64) * 512 < ((size_t)1 << 32),
+              "grid within HIP's limit");
+static_assert((size_t)linear_mfma_max_tokens(128, 8192) * 8192 * 2 <= ((size_t)1 << 32), "x within 32-bit offsets");
+
 hipError_t launch_linear_mfma(const uint8_t* tiles, int fmt, int M, int K, const uint16_t* x, int T, uint16_t* y,
                               hipStream_t st) {
-  LinMfmaArgs a{tiles, M, K, T, x, y, 0, 0};
-  return fmt == RMOE_FMT_BFP16 ? pick<RMOE_FMT_BFP16>(a, st) : pick<RMOE_FMT_Q4NX>(a, st);
+  // A token's bytes do not depend on its batch: one too large for a launch is several.
+  const int rows = linear_mfma_max_tokens(M, K);
+  for (int t0 = 0; t0 < T; t0 += std::min(rows, T - t0)) {
+    LinMfmaArgs a{tiles, M, K, std::min(rows, T - t0), x + (size_t)t0 * K, y + (size_t)t0 * M, 0, 0};
+    const hipError_t e = fmt == RMOE_FMT_BFP16 ? pick<RMOE_FMT_BFP16>(a, st) : pick<RMOE_FMT_Q4NX>(a, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace rmoe

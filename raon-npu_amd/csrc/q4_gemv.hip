@@ -192,7 +192,7 @@ hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, 
     else hipLaunchKernelGGL(linear_lane_kernel<32>, grid, block, 0, st, a);
     return hipGetLastError();
   }
-  if (linear_mfma_ok(M, K, x, T)) return launch_linear_mfma(tiles, RMOE_FMT_Q4NX, M, K, x, T, y, st);
+  if (linear_mfma_ok(x)) return launch_linear_mfma(tiles, RMOE_FMT_Q4NX, M, K, x, T, y, st);
   // The other operands (x at an address the MFMA kernel cannot load from).
   // Up to 4 K tiles per workgroup (one per wave); tall matrices, whose row bands alone
   // fill the chip, split K less (down to one workgroup per band) and skip the partials.

@@ -445,7 +445,14 @@ hipError_t launch_linear(const uint8_t* tiles, int M, int K, const uint16_t* x, 
                          RmoeScratch& s, hipStream_t st);
 
 // Both formats on MFMA (linear_mfma.hip), for the operands linear_mfma_ok() accepts.
-bool linear_mfma_ok(int M, int K, const uint16_t* x, int T);
+bool linear_mfma_ok(const uint16_t* x);
+// Most tokens of one launch: 32-bit byte offsets into x, and fewer than 2^32 threads in the
+// grid (up to 512 of them per 32 x 64 tile, which every batch near that size takes).
+constexpr int linear_mfma_max_tokens(int M, int K) {
+  const size_t by_x = ((size_t)1 << 32) / (2 * (size_t)K), by_grid = ((size_t)1 << 33) / (size_t)M;
+  const size_t n = (by_x < by_grid ? by_x : by_grid) / 32 * 32;
+  return n > 32 ? (int)n : 32;
+}
 hipError_t linear_mfma_setup();  // once per device before the first call
 hipError_t launch_linear_mfma(const uint8_t* tiles, int fmt, int M, int K, const uint16_t* x, int T, uint16_t* y,
                               hipStream_t st);

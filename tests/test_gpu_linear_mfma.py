@@ -89,6 +89,30 @@ def test_operands_at_odd_addresses(gpu_ctx, fmt, T):
     mat.free()
 
 
+@pytest.mark.parametrize("fmt", ["q4nx", "bfp16"])
+def test_batch_larger_than_one_launch(gpu_ctx, fmt):
+    """x of more than 4 GiB runs as several launches: every row as in batches of 65,536 tokens."""
+    import torch
+
+    K, T = 8192, 262144 + 77
+    mat, _, _ = _matrix(gpu_ctx, fmt, 128, K, 13)
+    mat.reserve(T)
+    g = torch.Generator(device="cuda").manual_seed(14)
+    x = torch.empty(T, K, dtype=torch.int16, device="cuda")
+    for t0 in range(0, T, 65536):
+        rows = x[t0:t0 + 65536]
+        rows.copy_(torch.randn(rows.shape, device="cuda", generator=g).to(torch.bfloat16).view(torch.int16))
+    y, want = (torch.zeros(T, 128, dtype=torch.int16, device="cuda") for _ in range(2))
+    st = torch.cuda.current_stream()
+    mat.linear_dev(x, T, y, stream=st)
+    for t0 in range(0, T, 65536):
+        n = min(65536, T - t0)
+        mat.linear_dev(x[t0:t0 + n], n, want[t0:t0 + n], stream=st)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want) and bool((y != 0).any(1).all())
+    mat.free()
+
+
 def test_non_finite_rows_stay_in_their_row(gpu_ctx):
     """Rows of x with an infinity or a NaN are not finite; the other rows of the tile are as without them."""
     for fmt in ("q4nx", "bfp16"):

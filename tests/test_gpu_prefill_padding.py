@@ -3,8 +3,10 @@
 The gate/up GEMM's last n-tile clears a row's columns past I, their group sums and the
 exponents of the chunks past the last live one; the combine takes one workgroup of
 H / 8 threads per token.  Down weights that are not zero past I make whatever stands there
-visible: each result is computed again after a call that leaves large values in the whole
-scratch, and compared with the oracle over weights cut at I."""
+visible: the columns and exponents to both formats, the group sums to the q4nx down, whose
+scales and mins multiply the sums of all groups.  Each result is computed again after a call
+that leaves large values in the whole scratch, and compared with the oracle over weights cut
+at I."""
 
 from __future__ import annotations
 
@@ -16,6 +18,7 @@ from raon_npu_amd import geometry as G
 from moe_fixtures import compare_bf16, make_layer, random_tokens
 from oracle import bfp16 as B
 from oracle import moe as om
+from oracle.q4nx import pack_gemv, quantize
 
 pytestmark = pytest.mark.gpu
 
@@ -24,22 +27,34 @@ pytestmark = pytest.mark.gpu
 # of the line between the two grouped kernels (46 rows per expert).
 @pytest.mark.parametrize("inter", [64, 320, 448])
 @pytest.mark.parametrize("T", [3, 300])
-def test_padding_is_cleared_on_every_call(gpu_ctx, inter, T):
+@pytest.mark.parametrize("layout", ["weights-d", "q4nx"])
+def test_padding_is_cleared_on_every_call(gpu_ctx, inter, T, layout):
     geom = G.MoeGeometry(hidden=256, inter=inter, n_routed=8, n_shared=1, top_k=2)
     full = G.MoeGeometry(hidden=256, inter=geom.inter_pad, n_routed=8, n_shared=1, top_k=2)
     rng = np.random.default_rng(81)
     downs = rng.normal(0.0, 0.02, (9, 256, geom.inter_pad)).astype(np.float32)
+
+    def pack(mats):
+        return b"".join(B.pack_gemv(m) if layout == "weights-d" else bytes(pack_gemv(*quantize(m))) for m in mats)
+
     lyrs = []
     for i, g in enumerate((geom, full)):
         syn = make_layer(g, seed=82 + i)
-        lyr = gpu_ctx.create_layer_d(1710 + i, g)
-        b1 = syn.gate_up[: 8 * g.gu_bytes]
-        lyr.upload_d(1, 0, b1)
-        lyr.upload_d(2, 0, b"".join(B.pack_gemv(m) for m in downs))
-        lyrs.append((lyr, b1))
+        if layout == "weights-d":
+            lyr = gpu_ctx.create_layer_d(1710 + i, g)
+            lyr.upload_d(1, 0, syn.gate_up[: 8 * g.gu_bytes])
+            lyr.upload_d(2, 0, pack(downs))
+        else:
+            lyr = gpu_ctx.create_layer(1710 + i, g)
+            lyr.upload_experts(syn.gate_up, pack(downs))
+        lyrs.append((lyr, syn.gate_up))
     cut = downs.copy()
-    cut[:, :, inter:] = 0.0
-    bank = om.DExpertBank(lyrs[0][1], b"".join(B.pack_gemv(m) for m in cut), 8, 256, inter)
+    cut[:, :, inter:] = 0.0  # I % 64 == 0: whole groups and blocks, the others keep their bytes
+    gate_up = lyrs[0][1]
+    if layout == "weights-d":
+        bank = om.DExpertBank(gate_up[: 8 * geom.gu_bytes], pack(cut), 8, 256, inter)
+    else:
+        bank = om.ExpertBank(gate_up, pack(cut), 9, 256, inter)
     ids = np.stack([rng.choice(8, 2, replace=False) for _ in range(T)]).astype(np.int32)
     wts = rng.uniform(0.1, 0.9, ids.shape).astype(np.float32)
     x = random_tokens(T, 256, 84)

@@ -884,6 +884,9 @@ static int set_router_common(rmoe_ctx* ctx, RmoeLayer* L, const void* w, bool w_
   HIP_TRY(hipSetDevice(ctx->device));
   const size_t wb = (size_t)L->n_routed * L->H * 2;
   if (!L->router_w && hipMalloc((void**)&L->router_w, wb) != hipSuccess) return fail(RMOE_ENOMEM, "hipMalloc failed");
+  // The context's stream is ordered with no other: whatever the caller queued that writes w
+  // has to end before it is read (the call takes no stream).
+  if (w_on_device) HIP_TRY(hipDeviceSynchronize());
   HIP_TRY(hipMemcpyAsync(L->router_w, w, wb, w_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
   if (bias) {
     if (!L->router_bias && hipMalloc((void**)&L->router_bias, L->n_routed * sizeof(float)) != hipSuccess)

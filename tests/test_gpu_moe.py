@@ -599,3 +599,24 @@ def test_grouped_dev_out_of_range_id(baseline, gpu_ctx):
     gpu_ctx.synchronize()
     np.testing.assert_array_equal(r_bad, r_ok)
     np.testing.assert_array_equal(s_bad, s_ok)
+
+
+def test_router_from_a_tensor_still_being_written(gpu_ctx):
+    """set_router of a device tensor takes no stream: work queued on any stream before the call,
+    here 50 ms of it ahead of the copy that fills the tensor, is in the weights."""
+    import torch
+
+    geom = G.MoeGeometry(hidden=256, inter=64, n_routed=16, n_shared=1, top_k=4)
+    syn = make_layer(geom, seed=301)
+    lyr = gpu_ctx.create_layer(301, geom)
+    want = torch.from_numpy(syn.router.view(np.int16)).cuda()
+    rw = torch.zeros_like(want)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(100_000_000)
+    rw.copy_(want)
+    lyr.set_router(rw, score="softmax")
+    ids, _, _ = lyr.route(random_tokens(8, 256, 302))
+    torch.cuda.synchronize()
+    lyr.set_router(syn.router, score="softmax")
+    np.testing.assert_array_equal(ids, lyr.route(random_tokens(8, 256, 302))[0])
+    lyr.free()

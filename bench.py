@@ -40,8 +40,8 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 # child `bench.py --profile-pass` runs, calibrated against a 512 MiB copy).  These are the
 # figures of the committed counter profile (profiles/decode_prefill_hbm_counters.txt),
 # reported instead only when rocprofv3 is absent, a pass fails, or --no-traffic is given.
-DECODE_TRAFFIC_BYTES = 1338163081
-LM_HEAD_TRAFFIC_BYTES = 749714547
+DECODE_TRAFFIC_BYTES = 1338580290
+LM_HEAD_TRAFFIC_BYTES = 769758695
 
 
 def log(msg: str) -> None:
@@ -259,7 +259,7 @@ def roofline(bound: str, work: float, seconds: float, kernel: str, per: str, tra
 # `bench.py --profile-configs`, calibrated against a 512 MiB copy).  These are the figures
 # of the committed counter profile (profiles/configs123_hbm_counters.txt), reported instead
 # only when rocprofv3 is absent, a pass fails, or --no-traffic is given.
-CONFIG_TRAFFIC_BYTES = {"config1_gemv": 1059270, "config2_decode_layer": 28544825, "config3_prefill_445": 466689316}
+CONFIG_TRAFFIC_BYTES = {"config1_gemv": 1059268, "config2_decode_layer": 28544658, "config3_prefill_445": 468116299}
 
 
 class ConfigWorkloads:
@@ -274,7 +274,7 @@ class ConfigWorkloads:
         gen = torch.Generator(device="cuda").manual_seed(seed + 21)
         # config 1: one q4nx GEMV, W [768, 2048] (the down width of a BASELINE expert), x 1 x 2048
         w = torch.randn(768, 2048, device="cuda", generator=gen) * 0.02
-        self.mat = ctx.quantize_matrix(w, 768, 2048)
+        self.mat = ctx.quantize_matrix(w, 768, 2048, stream=torch.cuda.current_stream())
         del w
         self.mat.reserve(1)
         self.x = torch.randn(1, 2048, device="cuda", generator=gen).to(torch.bfloat16).view(torch.int16)

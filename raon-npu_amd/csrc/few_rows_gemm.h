@@ -15,9 +15,9 @@
 // a CU, and the first block of them is requested with the first codes, before the row indices
 // are known.
 // Kernel times against grouped_gemm_kernel, gate/up and down: H=2048, I=768, 445 tokens 95 ->
-// 80 and 57 -> 47 us; H=2560, I=1088, 32 tokens 108 -> 79 and 61 -> 44 us, 256 tokens 142 ->
-// 119 and (bfp16) 139 -> 104 us: 4.2 to 4.9 TB/s of expert weights over the whole kernel.  The
-// rest is the workgroups' last round: 828 of them in 512 places at 445 tokens.  Tiles of 32
+// 76 and 57 -> 46 us, which is 3.4 and 2.8 TB/s of expert weights; H=2560, I=1088, 32 tokens
+// 108 -> 79 and 61 -> 51 us, 256 tokens 142 -> 105 and (bfp16) 139 -> 99 us, 4.2 and 4.8 TB/s.
+// The rest is the workgroups' last round: 828 of them in 512 places at 445 tokens.  Tiles of 32
 // rows instead of 48 cost 3 to 8 % at 445 tokens, three workgroups per CU (168 registers,
 // spills) 10 to 30 %, the first weight tiles requested after the correction instead of first
 // 5 to 45 %, weights three K steps ahead instead of two in the 16-row tiles 2 %.

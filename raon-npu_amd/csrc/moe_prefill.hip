@@ -433,8 +433,8 @@ __global__ __launch_bounds__(256) void router_prep_kernel(const uint16_t* __rest
 // ----------------------------------------------------------------- tile table --
 // One workgroup of 512 threads; thread e owns group e (routed 0..n_routed-1, shared
 // n_routed, whose rows start at shared_base).  (The dispatch scatter builds the same table
-// in its first workgroup when the groups fit its 256 threads; this kernel serves the other
-// cases and the table for a second GEMM with other shared rows.)
+// in a workgroup past its chunks when the groups fit its 256 threads; this kernel serves 256
+// routed experts and a shared one.)
 __global__ __launch_bounds__(512) void tile_table_kernel(const int32_t* __restrict__ offsets, int n_routed,
                                                          int shared_base, int shared_rows, uint32_t* __restrict__ tiles,
                                                          int* __restrict__ ntiles, int cap, int bm) {
@@ -1618,6 +1618,12 @@ hipError_t prefill_setup() {
 // of 128 experts: 8 tokens 71 / 88 us, 445 148 / 163, 640 (40 rows) 161 / 192, 800 (50) 206 /
 // 200, 1,024 248 / 236; H=2560, I=1088, 6 of 128: 300 tokens 214 / 259, 1,000 (47 rows) 346 /
 // 358, 2,000 576 / 560.
+// The average says little about a skewed batch, but both kernels take its hot experts in many
+// tiles.  Grouped calls by routing, few-rows / grouped_gemm_kernel: H=2048, I=768, 736 tokens
+// (46 rows) even 176 / 183 us, Zipf(1.1) 170 / 191, nine in ten routes on 16 experts 181 / 197,
+// all on the same 8 124 / 138; 796 tokens 180 / 194, 175 / 193, 188 / 197, 135 / 141.  H=2560,
+// I=1088, 981 tokens (46 rows) 289 / 305, 291 / 328, 307 / 348 and, all on the same 6, 212 /
+// 204; that routing loses at 445 tokens too, 122 / 111.
 constexpr int kFewRows = 46;
 static bool few_rows(const RmoeLayer& L, int T) {
   const size_t A = (size_t)T * L.top_k;

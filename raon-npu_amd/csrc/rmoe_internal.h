@@ -474,21 +474,21 @@ hipError_t launch_route(const RmoeLayer& L, const uint16_t* x, int T, int32_t* i
 // with its own copy of the one-token scratch.
 // out_routed (may be null) gets RTNE of the routed sum; out gets the full combine
 // (routed + shared, + x when residual).
-// n bytes (a multiple of 16) from src to dst, both 16-byte aligned and reachable by the device.
-hipError_t launch_copy16(const void* src, void* dst, size_t n, hipStream_t st);
 hipError_t launch_moe_decode(const RmoeLayer& L, const uint16_t* x, const int32_t* ids, const float* wts, int k,
                              bool with_shared, int act, float gb, float vb, bool residual, uint16_t* out,
                              uint16_t* out_routed, RmoeScratch& s, hipStream_t st, int stages = 3, int ntok = 1);
 
-// h[T, Ipad] = RTNE(act(gu[t, :I], gu[t, I:2I])) with zero columns [I, Ipad).
+// n bytes (a multiple of 16) from src to dst, both 16-byte aligned and reachable by the device.
+hipError_t launch_copy16(const void* src, void* dst, size_t n, hipStream_t st);
+
 // Assignments per dispatch chunk (per workgroup of the count and scatter kernels); the
 // chunk counts are counts[chunk][expert].
 constexpr int kDispatchChunk = 1024;
 // With counted, counts[][] already hold the chunk counts (the prefill top-k adds them) and
 // the count kernel is skipped.
-// With tiles != nullptr the first scatter workgroup also writes the grouped GEMM's tile
-// table (tiles of bm rows) for the routed groups plus, when shared_rows > 0, a shared group of that many rows
-// (n_experts + 1 <= 256 groups then).
+// With tiles != nullptr a workgroup of its own beside the scatter's writes the grouped GEMM's
+// tile table (tiles of bm rows) for the routed groups plus, when shared_rows > 0, a shared
+// group of that many rows (n_experts + 1 <= 256 groups then).
 hipError_t launch_dispatch(const int32_t* ids, int T, int k, int n_experts, int32_t* order, int32_t* inv,
                            int32_t* offsets, RmoeScratch& s, hipStream_t st, uint32_t* tiles = nullptr,
                            int* ntiles = nullptr, int cap = 0, int shared_rows = 0, bool counted = false,

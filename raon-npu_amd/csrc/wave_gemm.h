@@ -111,10 +111,6 @@ struct WaveRows {
   }
 };
 
-// acc += this wave's K tiles [kt0, kt1).  acc[m][f] in the MFMA output layout: lane (l16,
-// lq) holds activation rows 16m + 4lq + i (i = 0..3) of weight row l16 of fragment f.
-// The loads of tile kt + 1 are in flight under the MFMAs of tile kt (two register sets).
-// bfp16 sums are a quarter of the product's.
 // The int8 mantissas of two dwords times s (a power of two) as a bf16 operand, exactly: byte
 // u = m + 128 becomes the fp32 value 2^15 + u by one v_perm_b32, which minus 2^15 + 128 is
 // m.  (v_cvt_f32_i32 issues at a quarter of the rate of these.)
@@ -133,6 +129,10 @@ __device__ __forceinline__ uint4 b16_operand(uint32_t v0, uint32_t v1, float s) 
   return make_uint4(r[0], r[1], r[2], r[3]);
 }
 
+// acc += this wave's K tiles [kt0, kt1).  acc[m][f] in the MFMA output layout: lane (l16,
+// lq) holds activation rows 16m + 4lq + i (i = 0..3) of weight row l16 of fragment f.
+// The loads of tile kt + 1 are in flight under the MFMAs of tile kt (two register sets).
+// bfp16 sums are a quarter of the product's.
 template <int MF, int NF, int XI>
 __device__ __forceinline__ void wave_gemm_b16(const WaveOperands<MF, NF, XI>& o, int kt0, int kt1,
                                               wg_f32x4 (&acc)[MF][NF]) {

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the quantized-MoE hot path on one MI355X.
 
-Default workload: 48 stacked MoE layers of the BASELINE
+Default workload: 48 stacked MoE layers of the baseline
 shape (H=2048, I=768, 128 routed experts + 1 shared, softmax top-8, SwiGLU, q4nx
 weights N(0, 0.02)), residual add between layers, batch 1.  One step = one token
 through all 48 layers in ONE persistent launch (router on the device, 8 routed +
@@ -263,7 +263,7 @@ CONFIG_TRAFFIC_BYTES = {"config1_gemv": 1059268, "config2_decode_layer": 2854465
 
 
 class ConfigWorkloads:
-    """SURVEY configs 1-3 on the device: one q4nx GEMV [768, 2048] (config 1), one BASELINE
+    """Configs 1-3 on the device: one q4nx GEMV [768, 2048] (config 1), one BASELINE
     decode layer in a 1-layer persistent launch (config 2) and one BASELINE prefill layer of
     445 tokens (config 3), each a callable that queues one launch (sequence) on `stream`."""
 
@@ -299,7 +299,7 @@ class ConfigWorkloads:
     def config3(self):
         self.layer0.moe_prefill_dev(self.xp, self.T, self.op, stream=self.stream)
 
-    # algorithmic work per launch (SURVEY 8(d) figures)
+    # algorithmic work per launch
     CONFIG1_BYTES = 990208  # weights 983,040 + x 4,096 + y 3,072
 
     def config3_flops(self) -> int:
@@ -316,8 +316,7 @@ class ConfigWorkloads:
 
 
 def configs_bench(ctx, layers, geom, seed: int, stream, weights_d: bool = True) -> dict:
-    """SURVEY configs 1-3 (the other rows of the measurement table) and one weights-d MoE
-    layer at the released model's shapes; each timed as back-to-back launches in a graph,
+    """Configs 1-3 and one weights-d MoE layer at the released model's shapes; each timed as back-to-back launches in a graph,
     with its roofline block (algorithmic bytes or FLOPs over the measured time)."""
     import numpy as np
     import torch

@@ -6,8 +6,8 @@ Restates the NumPy host path of raon-npu for one mixture-of-experts layer:
 * ``situ_glu``      -- ``host/backend.py:47-62``
 * ``swiglu``        -- ``kernels/moe/reference.py:127-180`` (``gate_beta=None`` branch)
 * ``route_token``   -- ``host/raon.py:1224-1247`` (sigmoid + selection bias, the
-                       reference router) and the softmax router BASELINE.json's
-                       configs name (same steps with softmax scores)
+                       reference router) and the softmax router of the
+                       baseline geometry (same steps with softmax scores)
 * ``moe_experts``   -- ``host/backend.py:466-510`` (ascending expert id, fp32 sum)
 * ``moe_token``     -- ``host/raon.py:1288-1330`` (routed + shared, RTNE of the sum)
 * ``moe_experts_grouped`` -- the contract of ``npu/backend.py:4845-4979``:
@@ -102,7 +102,7 @@ class RouterSpec:
     """Router of one MoE layer.
 
     ``score`` is ``"sigmoid"`` (the reference router, ``host/raon.py:1233-1234``) or
-    ``"softmax"``.  ``bias`` is the selection-only
+    ``"softmax"`` (the baseline geometry).  ``bias`` is the selection-only
     ``e_score_correction_bias`` (``host/raon.py:1237``); ``renormalize`` and
     ``scaling`` follow ``host/raon.py:1242-1245``.
     """

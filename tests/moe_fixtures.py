@@ -1,4 +1,4 @@
-"""Seeded synthetic MoE layers for the parity tests (BASELINE.json config shapes).
+"""Seeded synthetic MoE layers for the parity tests.
 
 Weights are drawn N(0, std) in fp32, quantized and packed with the oracle's q4nx
 codec into the reference's bundle geometry (kernels/moe/pack.py: experts back to

@@ -41,7 +41,7 @@ def test_error_mapping_without_a_device():
 
 
 def test_geometry_matches_reference_constants():
-    # kernels/moe/pack.py:53-75 (reference model) and SURVEY/BASELINE byte counts.
+    # kernels/moe/pack.py:53-75 (reference model), byte counts of both geometries.
     assert RAON_1_MINI.gu_bytes == 3_481_600
     assert RAON_1_MINI.dn_bytes == 2_048_000
     assert RAON_1_MINI.inter_pad == 1280

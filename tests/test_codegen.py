@@ -90,7 +90,7 @@ def uncounted_load_hazards(asm_text: str, kernel_substr: str):
 
 
 def test_scanner_flags_a_copy_before_the_wait():
-    """The checker itself, on a hand-written fragment: a copy of a loaded register before
+    """The scanner itself, on a hand-written fragment: a copy of a loaded register before
     the wait is a hazard; the same copy after the wait is not."""
     head = "_ZN4rmoe19grouped_gemm_kernelE:\n\t;;#ASMSTART\n\tglobal_load_dwordx4 v[2:5], v[2:3], off\n\t;;#ASMEND\n"
     wait = "\t;;#ASMSTART\n\ts_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier\n\t;;#ASMEND\n"

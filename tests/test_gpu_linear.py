@@ -1,6 +1,6 @@
-"""GPU: dense q4nx GEMV (``linear``) vs the oracle (BASELINE config 1 and variants).
+"""GPU: dense q4nx GEMV (``linear``) vs the oracle ([768, 2048] and variants).
 
-Tolerance: max-abs 1e-2 and rel-L2 1e-3 against the fp32 oracle (BASELINE.json);
+Tolerance: max-abs 1e-2 and rel-L2 1e-3 against the fp32 oracle;
 additionally >= 99% of outputs must be bit-identical bf16 (the rest differ by
 fp32 summation order, one bf16 ulp).
 """
@@ -39,7 +39,7 @@ def _linear_dev(mat, x):
 
 
 def test_config1_gemv(gpu_ctx):
-    # BASELINE config 1: W 768x2048 N(0,0.02), x 1x2048 bf16 N(0,1), seed 0.
+    # W 768x2048 N(0,0.02), x 1x2048 bf16 N(0,1), seed 0.
     blob, wf, _ = _case(768, 2048, 0)
     rng = np.random.default_rng(0)
     x = f32_to_bf16(rng.standard_normal((1, 2048)).astype(np.float32))

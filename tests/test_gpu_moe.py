@@ -1,6 +1,6 @@
 """GPU: router, dispatch, decode MoE, grouped prefill and the residual stack vs the oracle.
 
-Bars (BASELINE.json): routing indices and dispatch permutations bit-exact; outputs
+Bars: routing indices and dispatch permutations bit-exact; outputs
 within max-abs 1e-2 and rel-L2 1e-3 of the fp32 oracle.  Routing exactness is
 asserted for every token whose k/k+1 selection-score gap exceeds 1e-6 (tokens
 closer than that are reported; fp32 summation order can legitimately reorder a

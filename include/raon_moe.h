@@ -81,7 +81,8 @@ void* rmoe_stream(rmoe_ctx* ctx);
  * upload of NpuBackend.preload / _get_weight_tensor (npu/backend.py:3265). */
 int rmoe_matrix_upload(rmoe_ctx* ctx, const void* pack_gemv_bytes, size_t nbytes, int M, int K, int* handle);
 /* Allocate an [M, K] matrix and fill it by quantizing fp32 device weights w_dev [M, K]
- * row-major on the device (quant/q4nx.py:127-200, bit-exact). */
+ * row-major on the device (quant/q4nx.py:127-200, bit-exact).  Synchronous; with stream NULL
+ * it first waits for whatever the device still runs, which may be writing the weights. */
 int rmoe_matrix_quantize_dev(rmoe_ctx* ctx, const float* w_dev, int M, int K, int* handle, void* stream);
 /* Read a matrix back as pack_gemv bytes (inverse re-layout; used for round trips). */
 int rmoe_matrix_download(rmoe_ctx* ctx, int handle, void* pack_gemv_bytes, size_t nbytes);
@@ -155,7 +156,8 @@ int rmoe_layer_upload_expert_q4k(rmoe_ctx* ctx, int layer, int expert, int part,
 #define RMOE_PART_GATE_UP 3
 int rmoe_layer_expert_matrix(rmoe_ctx* ctx, int layer, int expert, int part, int* handle);
 /* Quantize one expert from fp32 device weights (gate_up [2I, H], down [H, I] row-major;
- * the down input columns past I are zero-padded to Ipad).  Bit-exact quant/q4nx.py:127-200. */
+ * the down input columns past I are zero-padded to Ipad).  Bit-exact quant/q4nx.py:127-200.
+ * Synchronous; stream as in rmoe_matrix_quantize_dev. */
 int rmoe_layer_quantize_expert_dev(rmoe_ctx* ctx, int layer, int expert, const float* gate_up_dev,
                                    const float* down_dev, void* stream);
 /* Fill every expert of the layer with seeded synthetic weights N(0, std) generated on
@@ -191,7 +193,8 @@ int rmoe_layer_download_expert(rmoe_ctx* ctx, int layer, int expert, void* gate_
                                void* down, size_t dn_nbytes);
 /* Router of the layer (host/raon.py:1224-1247): weight bf16 [n_routed, H]; bias fp32
  * [n_routed] or NULL (selection-only e_score_correction_bias); score RMOE_SCORE_*;
- * renormalize 0/1; scaling = routed_scaling_factor. */
+ * renormalize 0/1; scaling = routed_scaling_factor.  Synchronous; the _dev form first waits
+ * for whatever the device still runs, which may be writing the weights. */
 int rmoe_layer_set_router(rmoe_ctx* ctx, int layer, const uint16_t* weight, const float* bias,
                           int score, int renormalize, float scaling);
 int rmoe_layer_set_router_dev(rmoe_ctx* ctx, int layer, const void* weight_dev, const float* bias_host,

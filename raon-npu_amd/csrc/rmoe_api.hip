@@ -518,6 +518,7 @@ int rmoe_matrix_quantize_dev(rmoe_ctx* ctx, const float* w_dev, int M, int K, in
   const size_t need = rmoe::matrix_bytes(M, K);
   if (hipMalloc((void**)&m.tiles, need) != hipSuccess) return fail(RMOE_ENOMEM, "hipMalloc of %zu bytes failed", need);
   hipStream_t st = pick_stream(ctx, stream);
+  if (!stream) HIP_TRY(hipDeviceSynchronize());  // the context's stream is ordered with no other
   HIP_TRY(rmoe::launch_quantize(w_dev, M, K, K, K, m.tiles, ctx->s.err, st));
   int r = sync_and_check(ctx, st);
   if (r != RMOE_OK) {
@@ -836,6 +837,7 @@ int rmoe_layer_quantize_expert_dev(rmoe_ctx* ctx, int layer, int expert, const f
   if (!gate_up_dev || !down_dev) return fail(RMOE_EINVAL, "null weights");
   HIP_TRY(hipSetDevice(ctx->device));
   hipStream_t st = pick_stream(ctx, stream);
+  if (!stream) HIP_TRY(hipDeviceSynchronize());  // the context's stream is ordered with no other
   HIP_TRY(rmoe::launch_quantize(gate_up_dev, 2 * L->I, L->H, L->H, L->H, L->gu + (size_t)expert * L->gu_bytes,
                                 ctx->s.err, st));
   HIP_TRY(rmoe::launch_quantize(down_dev, L->H, L->Ipad, L->I, L->I, L->dn + (size_t)expert * L->dn_bytes, ctx->s.err,

@@ -94,6 +94,33 @@ def test_quantize_and_download_tiles(gpu_ctx, M, K, offset):
     mat.free()
 
 
+def test_quantize_weights_still_being_written(gpu_ctx):
+    """Without a stream argument, quantizing waits for work queued on any stream before the call
+    (here 50 ms of it ahead of the copies that fill the weights)."""
+    import torch
+
+    import raon_npu_amd.geometry as G
+
+    rng = np.random.default_rng(61)
+    w = rng.normal(0.0, 0.02, (128, 256)).astype(np.float32)
+    want = pack_gemv(*quantize(w))
+    src = torch.from_numpy(w).cuda()
+    buf, gu = torch.zeros_like(src), torch.zeros_like(src)
+    dn = torch.zeros(256, 64, device="cuda")
+    lyr = gpu_ctx.create_layer(61, G.MoeGeometry(hidden=256, inter=64, n_routed=1, n_shared=0, top_k=1))
+    torch.cuda.synchronize()
+    torch.cuda._sleep(100_000_000)
+    buf.copy_(src)
+    mat = gpu_ctx.quantize_matrix(buf, 128, 256)
+    torch.cuda._sleep(100_000_000)
+    gu.copy_(src)
+    lyr.quantize_expert(0, gu, dn)
+    assert bytes(mat.download()) == bytes(want)
+    assert bytes(lyr.download_expert(0)[0]) == bytes(want)
+    mat.free()
+    lyr.free()
+
+
 # q4nx: 51 blocks of 10,240 bytes are one chunk of the download; 50, 52, 204 (the whole ring)
 # and 206 blocks.  bfp16: the same sizes at nine bits, chunks cut anywhere.
 @pytest.mark.parametrize("fmt, bits", [("q4nx", 5), ("bfp16", 9)])
